@@ -58,12 +58,12 @@ KERNEL_SOURCES = ("csrc/gates.hip", "csrc/launch_util.h", "csrc/kernels.h", "csr
 SLACK_DESC = {1: ", GCN products H.W^T truncated with the slack gate",
               2: ", GCN products and aggregations truncated with the slack gate",
               3: ", every layer truncation local (LocalARS, the reference's default truncation; not bit-exact)"}
-VALU_OPS_PER_AES = {"perm32x2_b512": 318, "perm64_b512": 390, "perm64_b1024": 390, "t4_rep32_b1024": 452}
+VALU_OPS_PER_AES = {"perm32x2_b512": 305, "perm64_b512": 390, "perm64_b1024": 390, "t4_rep32_b1024": 452}
 # The both-party form (one thread per element runs both parties' walks) issues
-# 617 VALU instructions per level loop of two AES calls on the T0/T1 table: a
+# 607 VALU instructions per level loop of two AES calls on the T0/T1 table: a
 # forward that mixes the two forms converts its AES calls at the lower count,
 # so its VALU rate is a lower bound.
-VALU_OPS_PER_AES_MIXED = dict(VALU_OPS_PER_AES, perm32x2_b512=308.5)
+VALU_OPS_PER_AES_MIXED = dict(VALU_OPS_PER_AES, perm32x2_b512=303.5)
 # LDS table bytes read per AES call: 16 four-byte lookups per round, ten rounds
 # (the same level-loop blocks: 160 ds_read_b32 in every variant)
 LDS_BYTES_PER_AES = 160 * 4

@@ -37,8 +37,10 @@ constexpr T0Table make_t0() {
 
 __device__ __constant__ const T0Table c_T0 = make_t0();
 
-__device__ __constant__ const AesRK c_rkH = aes_expand_c(kKeyHc);  // tree hash H
-__device__ __constant__ const AesRK c_rkL = aes_expand_c(kKeyLc);  // leaf hash HL
+// The fixed keys as compile-time constants: a round key is then an immediate move
+// into a scalar register where it is used, and holds none across a DCF level.
+constexpr AesRK c_rkH = aes_expand_c(kKeyHc);  // tree hash H
+constexpr AesRK c_rkL = aes_expand_c(kKeyLc);  // leaf hash HL
 
 __device__ __forceinline__ uint32_t rotl32(uint32_t v, int k) {
   return k == 0 ? v : ((v << k) | (v >> (32 - k)));
@@ -241,9 +243,9 @@ struct AesPerm {
 // Lane l reads copy l mod 32, so the two half-waves, which the LDS serves in
 // turn, never have two lanes on one bank.  One v_perm_b32 gives the address of
 // "T0[byte k of c]" (byte 0 = 4 (lane mod 32), byte 1 = byte k of c); T1 is the
-// same address plus the read's immediate offset 128.  A column is then
-// T0[a] ^ T1[b] ^ rotl(T0[c] ^ T1[d] ^ rotl(k, 16), 16): 4 address permutes, one
-// rotation and two three-input XORs (28 VALU per round against 36 with T0 alone).
+// same address plus the read's immediate offset 128.  A column is 4 address
+// permutes, one rotation and two three-input XORs (28 VALU per round against 36
+// with T0 alone).
 struct AesPerm2 {
   static constexpr int kWords = 256 * 64;
   static constexpr int kBytes = kWords * 4;
@@ -277,88 +279,113 @@ struct AesPerm2 {
   __device__ __forceinline__ uint32_t t1(uint32_t c) const {
     return *(const uint32_t *)(base + adr<K>(c) + 128);
   }
-  // rotl(T0[c] ^ T1[d] ^ rotl(k, 16), 16) = T2[c] ^ T3[d] ^ k; the round key is
-  // uniform, so its rotation is scalar work
-  __device__ __forceinline__ uint32_t col(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t k) const {
-    const uint32_t h = xor3(t0<2>(c), t1<3>(d), (k << 16) | (k >> 16));
-    return xor3(t0<0>(a), t1<1>(b), __builtin_amdgcn_alignbit(h, h, 16));
+  // The 16 table reads of a round by source column: T0[byte 0], T1[byte 1],
+  // T0[byte 2], T1[byte 3] of column j (the last round reads T0 throughout, whose
+  // byte 1 is S).
+  struct Reads {
+    uint32_t v[16];
+  };
+  template <bool LAST>
+  __device__ __forceinline__ void read(Reads &r, int j, uint32_t c) const {
+    r.v[4 * j] = t0<0>(c);
+    r.v[4 * j + 1] = LAST ? t0<1>(c) : t1<1>(c);
+    r.v[4 * j + 2] = t0<2>(c);
+    r.v[4 * j + 3] = LAST ? t0<3>(c) : t1<3>(c);
   }
-  // S[byte 0 of a] | S[byte 1 of b] << 8 | S[byte 2 of c] << 16 | S[byte 3 of d] << 24
-  // (S[x] is byte 1 of T0[x])
-  __device__ __forceinline__ uint32_t last(uint32_t a, uint32_t b, uint32_t c, uint32_t d) const {
-    const uint32_t lo = __builtin_amdgcn_perm(t0<1>(b), t0<0>(a), 0x0c0c0501u);
-    const uint32_t hi = __builtin_amdgcn_perm(t0<3>(d), t0<2>(c), 0x0c0c0501u);
+  // Column j of the round whose reads are r: T0[a] ^ T1[b] ^ rotl(T0[c] ^ T1[d] ^
+  // rotl(k, 16), 16), the second half being T2[c] ^ T3[d] ^ k; the round key is
+  // uniform, so its rotation is scalar work.
+  __device__ __forceinline__ static uint32_t col(const Reads &r, int j, uint32_t k) {
+    const uint32_t h = xor3(r.v[4 * ((j + 2) & 3) + 2], r.v[4 * ((j + 3) & 3) + 3], (k << 16) | (k >> 16));
+    return xor3(r.v[4 * j], r.v[4 * ((j + 1) & 3) + 1], __builtin_amdgcn_alignbit(h, h, 16));
+  }
+  // Column j of the last round before its key: S of byte i of column j + i
+  __device__ __forceinline__ static uint32_t last(const Reads &r, int j) {
+    const uint32_t lo = __builtin_amdgcn_perm(r.v[4 * ((j + 1) & 3) + 1], r.v[4 * j], 0x0c0c0501u);
+    const uint32_t hi = __builtin_amdgcn_perm(r.v[4 * ((j + 3) & 3) + 3], r.v[4 * ((j + 2) & 3) + 2], 0x0c0c0501u);
     return (hi << 16) | lo;
   }
-
-  __device__ __forceinline__ void rounds(uint32_t &c0, uint32_t &c1, uint32_t &c2, uint32_t &c3,
-                                         const AesRK &rk) const {
+  // Finishes round k from its reads and issues the reads of round k + 1.
+  __device__ __forceinline__ void step(Reads &r, const AesRK &rk, int k) const {
+    uint32_t c[4];
 #pragma unroll
-    for (int r = 1; r < 10; r++) {
-      const uint32_t n0 = col(c0, c1, c2, c3, rk.w[4 * r + 0]);
-      const uint32_t n1 = col(c1, c2, c3, c0, rk.w[4 * r + 1]);
-      const uint32_t n2 = col(c2, c3, c0, c1, rk.w[4 * r + 2]);
-      const uint32_t n3 = col(c3, c0, c1, c2, rk.w[4 * r + 3]);
-      c0 = n0;
-      c1 = n1;
-      c2 = n2;
-      c3 = n3;
+    for (int j = 0; j < 4; j++) c[j] = col(r, j, rk.w[4 * k + j]);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (k < 9)
+        read<false>(r, j, c[j]);
+      else
+        read<true>(r, j, c[j]);
+  }
+  // A round's 16 reads go out together, and the scheduler is held to that order:
+  // left to itself it keeps few reads in flight (a wait every 2.6 reads) and takes
+  // more registers for addresses formed early.  With two chains, one chain's reads
+  // are in flight while the other's columns are formed.  61 registers in the two-
+  // chain walk, so that two 1024-thread workgroups fit a CU: 105-106 G AES/s (348
+  // clocks per wave and AES, against 341 for its 160 reads) where the scheduler's
+  // own order ran 98 G in half the waves and 87-92 with one chain (walks of 25
+  // calls over 2^22 elements, both parties, correction words read from HBM).
+  __device__ __forceinline__ static void phase() { __builtin_amdgcn_sched_barrier(0); }
+
+  __device__ __forceinline__ void start(Reads &r, uint4 c) const {
+    read<false>(r, 0, c.x);
+    read<false>(r, 1, c.y);
+    read<false>(r, 2, c.z);
+    read<false>(r, 3, c.w);
+    phase();
+  }
+  // rounds 1..9 of the block whose first reads are r; then r holds the last round's
+  __device__ __forceinline__ void rounds(Reads &r, const AesRK &rk) const {
+#pragma unroll
+    for (int k = 1; k < 10; k++) {
+      step(r, rk, k);
+      phase();
     }
+  }
+  // two blocks, each under its own key
+  __device__ __forceinline__ void rounds2(Reads &a, const AesRK &ka, Reads &b, const AesRK &kb) const {
+#pragma unroll
+    for (int k = 1; k < 10; k++) {
+      step(a, ka, k);
+      phase();
+      step(b, kb, k);
+      phase();
+    }
+  }
+  __device__ __forceinline__ static uint4 whiten(uint4 in, const AesRK &rk) {
+    return make_uint4(in.x ^ rk.w[0], in.y ^ rk.w[1], in.z ^ rk.w[2], in.w ^ rk.w[3]);
+  }
+  __device__ __forceinline__ static uint4 enc_out(const Reads &r, const AesRK &rk) {
+    return make_uint4(last(r, 0) ^ rk.w[40], last(r, 1) ^ rk.w[41], last(r, 2) ^ rk.w[42], last(r, 3) ^ rk.w[43]);
+  }
+  // H(s) = AES_k(sigma(s)) ^ sigma(s), sigma(xL||xR) = (xL^xR)||xL, xR = words 0,1
+  __device__ __forceinline__ static uint4 hash_in(uint4 s, const AesRK &rk) {
+    return make_uint4(s.z ^ rk.w[0], s.w ^ rk.w[1], xor3(s.z, s.x, rk.w[2]), xor3(s.w, s.y, rk.w[3]));
+  }
+  __device__ __forceinline__ static uint4 hash_out(const Reads &r, const AesRK &rk, uint4 s) {
+    return make_uint4(xor3(last(r, 0), rk.w[40], s.z), xor3(last(r, 1), rk.w[41], s.w),
+                      xor3(last(r, 2), rk.w[42], s.z) ^ s.x, xor3(last(r, 3), rk.w[43], s.w) ^ s.y);
   }
 
   __device__ __forceinline__ uint4 enc(uint4 in, const AesRK &rk) const {
-    uint32_t c0 = in.x ^ rk.w[0], c1 = in.y ^ rk.w[1], c2 = in.z ^ rk.w[2], c3 = in.w ^ rk.w[3];
-    rounds(c0, c1, c2, c3, rk);
-    uint4 o;
-    o.x = last(c0, c1, c2, c3) ^ rk.w[40];
-    o.y = last(c1, c2, c3, c0) ^ rk.w[41];
-    o.z = last(c2, c3, c0, c1) ^ rk.w[42];
-    o.w = last(c3, c0, c1, c2) ^ rk.w[43];
-    return o;
+    Reads r;
+    start(r, whiten(in, rk));
+    rounds(r, rk);
+    return enc_out(r, rk);
   }
-
-  // H(s) = AES_k(sigma(s)) ^ sigma(s), sigma(xL||xR) = (xL^xR)||xL, xR = words 0,1
   __device__ __forceinline__ uint4 hash(uint4 s, const AesRK &rk) const {
-    uint32_t c0 = s.z ^ rk.w[0], c1 = s.w ^ rk.w[1];
-    uint32_t c2 = xor3(s.z, s.x, rk.w[2]), c3 = xor3(s.w, s.y, rk.w[3]);
-    rounds(c0, c1, c2, c3, rk);
-    uint4 o;
-    o.x = xor3(last(c0, c1, c2, c3), rk.w[40], s.z);
-    o.y = xor3(last(c1, c2, c3, c0), rk.w[41], s.w);
-    o.z = xor3(last(c2, c3, c0, c1), rk.w[42], s.z) ^ s.x;
-    o.w = xor3(last(c3, c0, c1, c2), rk.w[43], s.w) ^ s.y;
-    return o;
+    Reads r;
+    start(r, hash_in(s, rk));
+    rounds(r, rk);
+    return hash_out(r, rk, s);
   }
-
-  // hash of two independent blocks, their rounds side by side: one thread's
-  // two AES chains give the scheduler table reads of one to issue while the
-  // other's XORs wait
   __device__ __forceinline__ void hash2(uint4 s, uint4 u, const AesRK &rk, uint4 *hs, uint4 *hu) const {
-    uint32_t a0 = s.z ^ rk.w[0], a1 = s.w ^ rk.w[1];
-    uint32_t a2 = xor3(s.z, s.x, rk.w[2]), a3 = xor3(s.w, s.y, rk.w[3]);
-    uint32_t b0 = u.z ^ rk.w[0], b1 = u.w ^ rk.w[1];
-    uint32_t b2 = xor3(u.z, u.x, rk.w[2]), b3 = xor3(u.w, u.y, rk.w[3]);
-#pragma unroll
-    for (int r = 1; r < 10; r++) {
-      const uint32_t n0 = col(a0, a1, a2, a3, rk.w[4 * r + 0]);
-      const uint32_t m0 = col(b0, b1, b2, b3, rk.w[4 * r + 0]);
-      const uint32_t n1 = col(a1, a2, a3, a0, rk.w[4 * r + 1]);
-      const uint32_t m1 = col(b1, b2, b3, b0, rk.w[4 * r + 1]);
-      const uint32_t n2 = col(a2, a3, a0, a1, rk.w[4 * r + 2]);
-      const uint32_t m2 = col(b2, b3, b0, b1, rk.w[4 * r + 2]);
-      const uint32_t n3 = col(a3, a0, a1, a2, rk.w[4 * r + 3]);
-      const uint32_t m3 = col(b3, b0, b1, b2, rk.w[4 * r + 3]);
-      a0 = n0, a1 = n1, a2 = n2, a3 = n3;
-      b0 = m0, b1 = m1, b2 = m2, b3 = m3;
-    }
-    hs->x = xor3(last(a0, a1, a2, a3), rk.w[40], s.z);
-    hu->x = xor3(last(b0, b1, b2, b3), rk.w[40], u.z);
-    hs->y = xor3(last(a1, a2, a3, a0), rk.w[41], s.w);
-    hu->y = xor3(last(b1, b2, b3, b0), rk.w[41], u.w);
-    hs->z = xor3(last(a2, a3, a0, a1), rk.w[42], s.z) ^ s.x;
-    hu->z = xor3(last(b2, b3, b0, b1), rk.w[42], u.z) ^ u.x;
-    hs->w = xor3(last(a3, a0, a1, a2), rk.w[43], s.w) ^ s.y;
-    hu->w = xor3(last(b3, b0, b1, b2), rk.w[43], u.w) ^ u.y;
+    Reads a, b;
+    start(a, hash_in(s, rk));
+    start(b, hash_in(u, rk));
+    rounds2(a, rk, b, rk);
+    *hs = hash_out(a, rk, s);
+    *hu = hash_out(b, rk, u);
   }
 
   // Dealer PRF block AES_kd(idx_lo, idx_hi, field, gate).

@@ -18,31 +18,64 @@
 
 namespace mpcx {
 
-template <class A>
-__device__ __forceinline__ uint32_t dcf_eval_walk(const A &aes, uint4 s,
-                                                  int m, int L, const uint4 *__restrict__ cw, size_t stride,
-                                                  uint4 leaf, uint64_t x) {
-  uint32_t t = s.x & 1u, out = 0;
-  uint4 cnext = L > 0 ? cw[0] : make_uint4(0, 0, 0, 0);
-  // the path bits of x, MSB first: levels consume x >> (m-1-l); for m <= 32 the
-  // walk stays in 32-bit registers
-  const bool wide = m > 32;
-  const uint32_t xlo = uint32_t(x);
-  for (int l = 0; l < L; l++) {
-    const uint4 c = cnext;
-    if (l + 1 < L) cnext = cw[size_t(l + 1) * stride];
-    const int sh = m - 1 - l;
-    const uint32_t bit = wide ? uint32_t(x >> sh) & 1u : (xlo >> sh) & 1u;
-    const uint4 h = aes.hash(s, c_rkH);
-    const uint4 sl = xor_and4(h, c, 0u - t);
-    const uint32_t tl = sl.x & 1u;
-    out ^= (bit ^ 1u) & (tl ^ t);
-    s = xor_and4(sl, s, 0u - bit);
-    t = tl ^ (t & bit);
+
+// A 16-byte word of a key plane: base is uniform over the workgroup (a scalar
+// register pair), off a thread's 32-bit byte offset, so a load carries one
+// address register per lane.
+__device__ __forceinline__ uint4 ld16(const uint8_t *base, uint32_t off) {
+  return *reinterpret_cast<const uint4 *>(base + off);
+}
+
+// The planes of a DCF key at a workgroup's tile: pointers to the tile's first
+// element, and the distance of two levels' correction words in bytes.
+struct DcfTile {
+  const uint8_t *cw, *leaf;
+  size_t stride;
+};
+
+// All ones where bit k of v is set.
+__device__ __forceinline__ uint32_t bit_mask(uint32_t v, int k) {
+  return uint32_t(__builtin_amdgcn_sbfe(int(v), uint32_t(k), 1u));
+}
+// The path bits of an m-bit x left-aligned: the sign bit is the next level's, and
+// after the levels the low 7 bits of x (all of it for m < 7) are on top.
+template <typename X>
+struct PathBits {
+  X v;
+  __device__ __forceinline__ PathBits(X x, int m) : v(X(x << (int(8 * sizeof(X)) - m))) {}
+  __device__ __forceinline__ uint32_t next() {  // mask of the level's bit
+    const uint32_t r = uint32_t(int32_t(uint32_t(v >> (8 * sizeof(X) - 32))) >> 31);
+    v = X(v << 1);
+    return r;
   }
-  const uint4 lb = xor_and4(aes.hash(s, c_rkL), leaf, 0u - t);
-  const uint32_t pos = m >= 7 ? uint32_t(x & 127u) : uint32_t(x);
-  return out ^ parity_above(lb, pos);
+  __device__ __forceinline__ uint32_t leaf_pos(int m) const { return uint32_t(v >> (int(8 * sizeof(X)) - (m < 7 ? m : 7))); }
+};
+// (a ^ b) & ~m and a ^ (b & m) as one v_bitop3_b32 each
+__device__ __forceinline__ uint32_t xor_andn(uint32_t a, uint32_t b, uint32_t m) {
+  return __builtin_amdgcn_bitop3_b32(a, b, m, 0x14);
+}
+
+// One party's walk: s the party's root; t and the path bits are kept as masks.
+// A level's correction word is loaded at its start and used after its hash, some
+// thousand clocks later, so none is held a level ahead.
+template <class A, typename X>
+__device__ __forceinline__ uint32_t dcf_eval_walk(const A &aes, uint4 s, int m, int L, const DcfTile &k, uint32_t off,
+                                                  X x) {
+  uint32_t t = bit_mask(s.x, 0), out = 0;
+  PathBits<X> path(x, m);
+  const uint8_t *cw = k.cw;
+  for (int l = 0; l < L; l++, cw += k.stride) {
+    const uint4 c = ld16(cw, off);
+    const uint32_t bit = path.next();
+    const uint4 sl = xor_and4(aes.hash(s, c_rkH), c, t);
+    const uint32_t tl = bit_mask(sl.x, 0);
+    out ^= xor_andn(tl, t, bit);
+    s = xor_and4(sl, s, bit);
+    t = xor_and(tl, t, bit);
+  }
+  const uint4 leaf = ld16(k.leaf, off);
+  const uint4 lb = xor_and4(aes.hash(s, c_rkL), leaf, t);
+  return (out & 1u) ^ parity_above(lb, path.leaf_pos(m));
 }
 
 // Both parties' hashes of a level: side by side on the T0/T1 table, one after
@@ -61,34 +94,30 @@ __device__ __forceinline__ void hash_pair(const A &aes, uint4 s, uint4 u, const 
 // (the correction words and the leaf are common to the two keys): the XOR of
 // the two parties' outputs, i.e. the reconstructed bit.  Each level hashes the
 // two seeds side by side and reads its correction word once.
-template <class A>
-__device__ __forceinline__ uint32_t dcf_eval_walk2(const A &aes, uint4 s0, uint4 s1, int m, int L,
-                                                   const uint4 *__restrict__ cw, size_t stride, uint4 leaf,
-                                                   uint64_t x) {
-  uint32_t t0 = s0.x & 1u, t1 = s1.x & 1u, out = 0;
-  uint4 cnext = L > 0 ? cw[0] : make_uint4(0, 0, 0, 0);
-  const bool wide = m > 32;
-  const uint32_t xlo = uint32_t(x);
-  for (int l = 0; l < L; l++) {
-    const uint4 c = cnext;
-    if (l + 1 < L) cnext = cw[size_t(l + 1) * stride];
-    const int sh = m - 1 - l;
-    const uint32_t bit = wide ? uint32_t(x >> sh) & 1u : (xlo >> sh) & 1u;
+template <class A, typename X>
+__device__ __forceinline__ uint32_t dcf_eval_walk2(const A &aes, uint4 s0, uint4 s1, int m, int L, const DcfTile &k,
+                                                   uint32_t off, X x) {
+  uint32_t t0 = bit_mask(s0.x, 0), t1 = bit_mask(s1.x, 0), out = 0;
+  PathBits<X> path(x, m);
+  const uint8_t *cw = k.cw;
+  for (int l = 0; l < L; l++, cw += k.stride) {
+    const uint4 c = ld16(cw, off);
+    const uint32_t bit = path.next();
     uint4 h0, h1;
     hash_pair(aes, s0, s1, c_rkH, &h0, &h1);
-    const uint4 sl0 = xor_and4(h0, c, 0u - t0), sl1 = xor_and4(h1, c, 0u - t1);
-    const uint32_t tl0 = sl0.x & 1u, tl1 = sl1.x & 1u;
-    out ^= (bit ^ 1u) & (tl0 ^ t0 ^ tl1 ^ t1);
-    s0 = xor_and4(sl0, s0, 0u - bit);
-    s1 = xor_and4(sl1, s1, 0u - bit);
-    t0 = tl0 ^ (t0 & bit);
-    t1 = tl1 ^ (t1 & bit);
+    const uint4 sl0 = xor_and4(h0, c, t0), sl1 = xor_and4(h1, c, t1);
+    const uint32_t tl0 = bit_mask(sl0.x, 0), tl1 = bit_mask(sl1.x, 0);
+    out ^= xor_andn(tl0 ^ tl1, t0 ^ t1, bit);
+    s0 = xor_and4(sl0, s0, bit);
+    s1 = xor_and4(sl1, s1, bit);
+    t0 = xor_and(tl0, t0, bit);
+    t1 = xor_and(tl1, t1, bit);
   }
+  const uint4 leaf = ld16(k.leaf, off);
   uint4 l0, l1;
   hash_pair(aes, s0, s1, c_rkL, &l0, &l1);
-  const uint4 lb = xor4(xor_and4(l0, leaf, 0u - t0), xor_and4(l1, leaf, 0u - t1));
-  const uint32_t pos = m >= 7 ? uint32_t(x & 127u) : uint32_t(x);
-  return out ^ parity_above(lb, pos);
+  const uint4 lb = xor4(xor_and4(l0, leaf, t0), xor_and4(l1, leaf, t1));
+  return (out & 1u) ^ parity_above(lb, path.leaf_pos(m));
 }
 
 // The same walk on the quad-lane AES (latency-bound launches): lane j of a quad

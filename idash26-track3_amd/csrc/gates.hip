@@ -98,27 +98,35 @@ __device__ __forceinline__ T tr_shifted_input(const TrArgs<T> &a, size_t i, T xh
   return low_bits<T>(x + (T(1) << a.sb), a.m);
 }
 
-// Party p's masked DCF output bits of element i (the gate's planes a and b):
-// the DCF walks over the shifted input xp with the party's roots and mask bits
-// (K) and the correction and leaf words, which are the same in both parties'
-// keys (KC: any party's copy).
+// A DCF's planes at a tile of elements from base on (KC: any party's key, the
+// correction and leaf words being the same in both), a party's root of the
+// tile's element e and its output-mask bit (base a multiple of 64).
+__device__ __forceinline__ DcfTile dcf_tile(const DcfLayout &d, const uint8_t *KC, size_t base, size_t N) {
+  return {KC + d.off_cw + 16 * base, KC + d.off_leaf + 16 * base, 16 * N};
+}
+__device__ __forceinline__ uint4 dcf_root(const DcfLayout &d, const uint8_t *K, size_t base, uint32_t e) {
+  return ld16(K + d.off_root + 16 * base, 16 * e);
+}
+__device__ __forceinline__ uint32_t dcf_zbit(const DcfLayout &d, const uint8_t *K, size_t base, uint32_t e) {
+  return (reinterpret_cast<const uint32_t *>(K + d.off_z + base / 8)[e >> 5] >> (e & 31u)) & 1u;
+}
+
+// Party p's masked DCF output bits of element base + e (the gate's planes a and
+// b): the DCF walks over the shifted input xp with the party's roots and mask
+// bits (K) and the shared correction and leaf words (KC).
 template <typename T, class Aes>
-__device__ __forceinline__ void tr_dcf_bits(Aes &aes, const TrArgs<T> &a, const uint8_t *K,
-                                            const uint8_t *KC, size_t i, T xp, uint32_t *ra, uint32_t *rb) {
+__device__ __forceinline__ void tr_dcf_bits(const Aes &aes, const TrArgs<T> &a, const uint8_t *K, const uint8_t *KC,
+                                            size_t base, uint32_t e, T xp, uint32_t *ra, uint32_t *rb) {
   const T lowmask = (T(1) << a.sb) - T(1);
   const T smask = (T(1) << a.s) - T(1);
-  if (a.use_a) {
-    *ra = dcf_eval_walk(aes, reinterpret_cast<const uint4 *>(K + a.a.off_root)[i], a.a.m, a.a.L,
-                        reinterpret_cast<const uint4 *>(KC + a.a.off_cw) + i, a.N,
-                        reinterpret_cast<const uint4 *>(KC + a.a.off_leaf)[i], uint64_t(xp & lowmask));
-    *ra ^= get_bit(reinterpret_cast<const uint64_t *>(K + a.a.off_z), i);
-  }
-  if (a.use_b) {
-    *rb = dcf_eval_walk(aes, reinterpret_cast<const uint4 *>(K + a.b.off_root)[i], a.b.m, a.b.L,
-                        reinterpret_cast<const uint4 *>(KC + a.b.off_cw) + i, a.N,
-                        reinterpret_cast<const uint4 *>(KC + a.b.off_leaf)[i], uint64_t(xp & smask));
-    *rb ^= get_bit(reinterpret_cast<const uint64_t *>(K + a.b.off_z), i);
-  }
+  if (a.use_a)
+    *ra = dcf_eval_walk(aes, dcf_root(a.a, K, base, e), a.a.m, a.a.L, dcf_tile(a.a, KC, base, a.N), 16 * e,
+                        T(xp & lowmask)) ^
+          dcf_zbit(a.a, K, base, e);
+  if (a.use_b)
+    *rb = dcf_eval_walk(aes, dcf_root(a.b, K, base, e), a.b.m, a.b.L, dcf_tile(a.b, KC, base, a.N), 16 * e,
+                        T(xp & smask)) ^
+          dcf_zbit(a.b, K, base, e);
 }
 
 // Party p's output message for element i once the masked DCF outputs are
@@ -180,19 +188,20 @@ struct TrXchg {
   T xm[2][kTrMaxTile];
 };
 
-// Gate a on element i of a tile (element e of the tile, wave wv of its party's
-// half, masked input xh): party p's DCF walks, the exchange of the masked DCF
+// Gate a on element e of the tile from base on (wave wv of its party's half,
+// masked input xh): party p's DCF walks, the exchange of the masked DCF
 // output bits, party p's output message, the exchange of the messages.  Every
 // thread of the workgroup calls it (the exchanges synchronise the workgroup);
-// it returns the revealed output of element i to both parties' threads.
+// it returns the revealed output of the element to both parties' threads.
 template <typename T, class Aes>
-__device__ __forceinline__ T tr_tile(Aes &aes, const TrArgs<T> &a, TrXchg<T> &x, int p, int e, int wv,
-                                     const uint8_t *K, const uint8_t *KC, size_t i, bool in, T xh) {
+__device__ __forceinline__ T tr_tile(const Aes &aes, const TrArgs<T> &a, TrXchg<T> &x, int p, uint32_t e, uint32_t wv,
+                                     const uint8_t *K, const uint8_t *KC, size_t base, bool in, T xh) {
   uint32_t ra = 0, rb = 0;
   T xp = 0;
+  const size_t i = base + e;
   if (in) {
     xp = tr_shifted_input(a, i, xh);
-    tr_dcf_bits(aes, a, K, KC, i, xp, &ra, &rb);
+    tr_dcf_bits(aes, a, K, KC, base, e, xp, &ra, &rb);
   }
   // exchange 1: the masked DCF output bits
   const uint64_t wa = __ballot(ra), wb = __ballot(rb);
@@ -223,9 +232,10 @@ __device__ __forceinline__ void tr_eval_tiles(const TrArgs<T> &a, const TrArgs<T
   AesLds<NT, REP>::fill(lds);
   AesLds<NT, REP> aes(lds);
   const int h = int(blockDim.x) / 2;
-  const int p = int(threadIdx.x) >= h ? 1 : 0;
-  const int e = int(threadIdx.x) - p * h;  // element of the tile
-  const int wv = e >> 6;                   // wave of the party's half
+  // a party's half is whole waves, so the party is uniform over a wave
+  const int p = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >= h ? 1 : 0);
+  const uint32_t e = threadIdx.x - uint32_t(p * h);  // element of the tile
+  const uint32_t wv = e >> 6;                        // wave of the party's half
   // The correction words and leaf words of a DCF key are the same for both
   // parties (public to both); both parties read party 0's planes, so one copy
   // serves the two evaluations (and a streamed arena moves it once).
@@ -245,8 +255,8 @@ __device__ __forceinline__ void tr_eval_tiles(const TrArgs<T> &a, const TrArgs<T
         xin = a.xhat[i];
       }
     }
-    T y = tr_tile(aes, a, x, p, e, wv, K, KC, i, in, xin);
-    if constexpr (TWO) y = tr_tile(aes, a2, x, p, e, wv, K, KC, i, in, y);
+    T y = tr_tile(aes, a, x, p, e, wv, K, KC, base, in, xin);
+    if constexpr (TWO) y = tr_tile(aes, a2, x, p, e, wv, K, KC, base, in, y);
     if (p == 0 && in) {
       if constexpr (POOL)
         q.vn[o] = v0 + y;
@@ -264,41 +274,40 @@ __device__ __forceinline__ void tr_eval_tiles(const TrArgs<T> &a, const TrArgs<T
 // sum of the two output messages, the revealed output.  The same keys and
 // algebra as tr_tile, with no exchange buffers and no barriers.
 template <typename T, class Aes>
-__device__ __forceinline__ T tr_both(const Aes &aes, const TrArgs<T> &a, size_t i, T xh) {
+__device__ __forceinline__ T tr_both(const Aes &aes, const TrArgs<T> &a, size_t base, uint32_t e, T xh) {
+  const size_t i = base + e;
   const T xp = tr_shifted_input(a, i, xh);
   const T lowmask = (T(1) << a.sb) - T(1);
   const T smask = (T(1) << a.s) - T(1);
   uint32_t bh = 0, dh = 0;
-  if (a.use_a) {
-    bh = dcf_eval_walk2(aes, reinterpret_cast<const uint4 *>(a.k0 + a.a.off_root)[i],
-                        reinterpret_cast<const uint4 *>(a.k1 + a.a.off_root)[i], a.a.m, a.a.L,
-                        reinterpret_cast<const uint4 *>(a.k0 + a.a.off_cw) + i, a.N,
-                        reinterpret_cast<const uint4 *>(a.k0 + a.a.off_leaf)[i], uint64_t(xp & lowmask));
-    bh ^= get_bit(reinterpret_cast<const uint64_t *>(a.k0 + a.a.off_z), i) ^
-          get_bit(reinterpret_cast<const uint64_t *>(a.k1 + a.a.off_z), i);
-  }
-  if (a.use_b) {
-    dh = dcf_eval_walk2(aes, reinterpret_cast<const uint4 *>(a.k0 + a.b.off_root)[i],
-                        reinterpret_cast<const uint4 *>(a.k1 + a.b.off_root)[i], a.b.m, a.b.L,
-                        reinterpret_cast<const uint4 *>(a.k0 + a.b.off_cw) + i, a.N,
-                        reinterpret_cast<const uint4 *>(a.k0 + a.b.off_leaf)[i], uint64_t(xp & smask));
-    dh ^= get_bit(reinterpret_cast<const uint64_t *>(a.k0 + a.b.off_z), i) ^
-          get_bit(reinterpret_cast<const uint64_t *>(a.k1 + a.b.off_z), i);
-  }
+  if (a.use_a)
+    bh = dcf_eval_walk2(aes, dcf_root(a.a, a.k0, base, e), dcf_root(a.a, a.k1, base, e), a.a.m, a.a.L,
+                        dcf_tile(a.a, a.k0, base, a.N), 16 * e, T(xp & lowmask)) ^
+         dcf_zbit(a.a, a.k0, base, e) ^ dcf_zbit(a.a, a.k1, base, e);
+  if (a.use_b)
+    dh = dcf_eval_walk2(aes, dcf_root(a.b, a.k0, base, e), dcf_root(a.b, a.k1, base, e), a.b.m, a.b.L,
+                        dcf_tile(a.b, a.k0, base, a.N), 16 * e, T(xp & smask)) ^
+         dcf_zbit(a.b, a.k0, base, e) ^ dcf_zbit(a.b, a.k1, base, e);
   const uint32_t hb = uint32_t(xp >> a.sb) & 1u;
   return tr_reveal_sum<T>(a, tr_out_share(a, 0, a.k0, i, xh, xp, hb, bh, dh),
                           tr_out_share(a, 1, a.k1, i, xh, xp, hb, bh, dh));
 }
 
-// The elements of a both-party launch, one per thread (grid-stride): gate a,
-// then (TWO) gate a2 on its revealed output, or (POOL) a max-pool level.
+// The elements of a both-party launch, one per thread: gate a, then (TWO) gate
+// a2 on its revealed output, or (POOL) a max-pool level.  Tiles of 64 elements
+// are dealt to the workgroups in turn, wave by wave, so that a last round that
+// does not fill the chip still puts about the same number of waves on every CU.
 template <typename T, int NT, int REP, bool TWO, bool POOL>
 __device__ __forceinline__ void tr_eval_both(const TrArgs<T> &a, const TrArgs<T> &a2, const TrPool<T> &q) {
   __shared__ __align__(16) uint32_t lds[AesLds<NT, REP>::kWords];
   AesLds<NT, REP>::fill(lds);
   const AesLds<NT, REP> aes(lds);
-  const size_t stride = size_t(gridDim.x) * blockDim.x;
-  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < a.N; i += stride) {
+  const uint32_t e = lane_id();
+  const size_t wave = size_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  const size_t stride = 64 * size_t(gridDim.x) * (blockDim.x >> 6);
+  for (size_t base = 64 * (wave * gridDim.x + blockIdx.x); base < a.N; base += stride) {
+    const size_t i = base + e;
+    if (i >= a.N) break;
     T xin, v0 = 0;
     uint32_t o = 0;
     if constexpr (POOL) {
@@ -308,8 +317,8 @@ __device__ __forceinline__ void tr_eval_both(const TrArgs<T> &a, const TrArgs<T>
     } else {
       xin = a.xhat[i];
     }
-    T y = tr_both(aes, a, i, xin);
-    if constexpr (TWO) y = tr_both(aes, a2, i, y);
+    T y = tr_both(aes, a, base, e, xin);
+    if constexpr (TWO) y = tr_both(aes, a2, base, e, y);
     if constexpr (POOL)
       q.vn[o] = v0 + y;
     else
@@ -517,8 +526,11 @@ __global__ void k_tr_eval_pool_tail_q(TrTail<T> t) {
   for (int k = int(threadIdx.x); k < nc; k += int(blockDim.x)) t.out[g0 + k] = vin[k * R0];
 }
 
+// 64 registers, so that two 1024-thread workgroups fit a CU where a launch takes
+// them (the rounds' reads go out in phases, AesPerm2, so fewer registers cost no
+// order of loads).
 template <typename T, int NT, int REP, int TAG>
-__global__ void k_tr_eval(TrArgs<T> a) {
+__global__ void __launch_bounds__(1024, 8) k_tr_eval(TrArgs<T> a) {
   if (a.prio) __builtin_amdgcn_s_setprio(2);
   tr_eval_tiles<T, NT, REP, false, false>(a, a, TrPool<T>{});
 }
@@ -541,15 +553,20 @@ __global__ void k_tr_eval2(TrArgs<T> a, TrArgs<T> a2) {
 }
 
 // Both-party forms: one thread per element for both parties.
-template <typename T, int NT, int REP, int TAG>
-__global__ void k_tr_eval_b(TrArgs<T> a) {
+template <typename T, int NT, int REP, int W, int TAG>
+__global__ void __launch_bounds__(1024, W) k_tr_eval_b(TrArgs<T> a) {
   if (a.prio) __builtin_amdgcn_s_setprio(2);
   tr_eval_both<T, NT, REP, false, false>(a, a, TrPool<T>{});
 }
-template <typename T, int NT, int REP, int TAG>
-__global__ void k_tr_eval2_b(TrArgs<T> a, TrArgs<T> a2) {
+template <typename T, int NT, int REP, int W, int TAG>
+__global__ void __launch_bounds__(1024, W) k_tr_eval2_b(TrArgs<T> a, TrArgs<T> a2) {
   if (a.prio) __builtin_amdgcn_s_setprio(2);
   tr_eval_both<T, NT, REP, true, false>(a, a2, TrPool<T>{});
+}
+template <typename T, int NT, int REP, int W, int TAG>
+__global__ void __launch_bounds__(1024, W) k_tr_eval_pool_b(TrArgs<T> a, TrPool<T> q) {
+  if (a.prio) __builtin_amdgcn_s_setprio(2);
+  tr_eval_both<T, NT, REP, false, true>(a, a, q);
 }
 
 // Party mode, phase 1: party p's masked DCF output bits (one ballot word per
@@ -561,14 +578,14 @@ __global__ void k_tr_party_bits(TrArgs<T> a, uint64_t *bits) {
   AesLds<NT, REP> aes(lds);
   const size_t W = (a.N + 63) / 64;
   const size_t stride = size_t(gridDim.x) * blockDim.x;
-  for (size_t base = size_t(blockIdx.x) * blockDim.x + (threadIdx.x & ~63u); base < a.N; base += stride) {
-    const size_t i = base + lane_id();
+  for (size_t base = size_t(blockIdx.x) * blockDim.x; base < a.N; base += stride) {
+    const size_t i = base + threadIdx.x;
     uint32_t ra = 0, rb = 0;
-    if (i < a.N) tr_dcf_bits(aes, a, a.k0, a.k0, i, tr_shifted_input(a, i, a.xhat[i]), &ra, &rb);
+    if (i < a.N) tr_dcf_bits(aes, a, a.k0, a.k0, base, threadIdx.x, tr_shifted_input(a, i, a.xhat[i]), &ra, &rb);
     const uint64_t wa = __ballot(ra), wb = __ballot(rb);
-    if (lane_id() == 0) {
-      if (a.use_a) bits[base >> 6] = wa;
-      if (a.use_b) bits[W + (base >> 6)] = wb;
+    if (lane_id() == 0 && i < a.N) {
+      if (a.use_a) bits[i >> 6] = wa;
+      if (a.use_b) bits[W + (i >> 6)] = wb;
     }
   }
 }
@@ -734,19 +751,17 @@ hipError_t launch_tr_keygen(const Launch &L, const TrLayout &lay, uint64_t seed,
   });
 }
 
-// Workgroup of a gate evaluation: the context's explicit size, else the
-// variant's; a launch of at least 2^22 elements on the default 512-thread
-// variant takes 1024 threads (one T-table per 16 waves).  Measured: 3.28
-// against 3.11 G DCF evals/s on 2^24 ReLUs, while the model's launches (up to
-// 10^6 elements) and the adjacency normalisation's (3.4 * 10^6) lose 6-10% at
-// 1024 and keep 512.
 // A gate evaluation of fewer elements than this is latency-bound (a few
 // thousand wavefronts of one dependent AES chain each) and sits on its lane's
 // critical path while other lanes' large gates fill the GPU: its waves take the
 // SIMDs' issue slots first.
 constexpr size_t kTrPrioN = size_t(1) << 17;
 // Threads per workgroup of the one-launch gate kernel (both parties' threads for
-// block/2 elements).  A small gate spreads over the CUs: with the variant's block
+// block/2 elements): the context's explicit size, else the variant's.  A launch
+// of at least 2048 elements per CU on the default 512-thread variant takes 1024
+// threads, two workgroups per CU: 64-bit RELUs of 2048, 4096 and 8192 elements
+// per CU 587, 1162 and 2320 us against 623, 1228 and 2440.  Beside other streams'
+// launches that starts at 2^22 elements.  A small gate spreads over the CUs: with the variant's block
 // its few workgroups put 8 waves on each CU they land on, and a CU's LDS serves
 // one 64-lane table read per two clocks, so every AES round of those waves waits
 // on one CU's LDS while the other CUs idle; about one workgroup per CU, of at
@@ -754,7 +769,7 @@ constexpr size_t kTrPrioN = size_t(1) << 17;
 static int tr_eval_block(const Launch &L, size_t n) {
   const int b = variant_block(L);
   if (L.aes_block != 0) return b;
-  if (b == 512 && n >= (size_t(1) << 22)) return 1024;
+  if (b == 512 && n >= (L.shared ? size_t(1) << 22 : 2048 * size_t(L.num_cu))) return 1024;
   if (!L.spread_small) return b;
   const size_t per_cu = (n + size_t(L.num_cu) - 1) / size_t(L.num_cu);
   const size_t h = std::max<size_t>(64, (per_cu + 63) / 64 * 64);
@@ -787,24 +802,31 @@ static int quad_grid(const Launch &L, size_t n) {
 }
 
 // The both-party form (one thread per element for both parties, 1024-thread
-// workgroups: one per CU at 68 VGPRs, 64 KiB of LDS) for gates of at most
-// L.both_aes AES calls per element and party over Z_2^32 (the launcher's only
-// instance), in launches of at least L.both_min elements per CU.  Interleaved
-// on one box against the one-lane kernel: affinity B = 64 in 3 lanes +4.6%
-// (gates up to 14 calls, 1024 elements per CU), in 1 lane -3.8% with gates up
-// to 14 calls and unchanged up to 6; adjacency normalisation B = 1024 (6-call
-// gates) +10% in 3 groups, +7.5% in one.  In lanes 512 elements per CU gains
-// again (B = 64 +1.4%, B = 32 +2.5%; 384 and 256 lose at B = 32).  Also
-// measured: every gate launch in this form (B = 64 -0.6%), 512, 768 and 896
-// threads, bw = 64 (2-3% slower), the 25-call RELU of 2^24 elements alone (6%
-// slower).  A truncation pair in this form (k_tr_eval2_b, lanes of at most 8
-// samples): B = 16 +4%, B = 24 +2%; a max-pool level in this form measured no
-// gain.
+// workgroups) for gates of at most L.both_aes AES calls per element and party
+// over Z_2^32, in launches of at least L.both_min elements per CU.  Its walks run
+// two AES chains a thread (AesPerm2::hash2) and read each correction word once,
+// for which the clock, bound by power, runs higher too: 4096 elements per CU of
+// a 25-call gate take 541 us, the one-lane kernel 558; 8192 1037 against 1088;
+// 16384 (2^22 ReLUs on 256 CUs) 1995, the one-lane kernel before its rounds were
+// held in phases 2270.  A truncation pair in this form (k_tr_eval2_b, lanes of at
+// most 8 samples): B = 16 +4%, B = 24 +2%.
 template <typename T>
 static int both_block(const Launch &L, const TrArgs<T> &a) {
+  if (sizeof(T) != 4) return 0;
   const int aes = (a.use_a ? a.a.L + 1 : 0) + (a.use_b ? a.b.L + 1 : 0);
   if (L.aes_block != 0 || aes > L.both_aes) return 0;
   return a.N >= size_t(L.num_cu) * size_t(L.both_min) ? 1024 : 0;
+}
+// Waves per SIMD of a both-party launch.  Eight (64 registers, a few spilled
+// outside the level loops; two workgroups per CU) keep the LDS reading at 98% of
+// its rate, but a round of the grid is then 2048 elements per CU: from 4096 on
+// that is worth it (8192 per CU: 1037 against 1072 us for four waves; 1536: 261
+// against 204).  Beside other streams' launches four (one workgroup per CU) leave
+// those the other half of the CU: affinity B = 64 in 3 lanes 5.17 against 5.27 ms,
+// adjacency normalisation B = 1024 1.50 against 1.53.
+template <typename T>
+static int both_waves(const Launch &L, const TrArgs<T> &a) {
+  return !L.shared && a.N >= 4096 * size_t(L.num_cu) ? 8 : 4;
 }
 
 // The kernel form of a gate evaluation outside the max-pool form: the
@@ -812,12 +834,26 @@ static int both_block(const Launch &L, const TrArgs<T> &a) {
 template <typename T>
 static int tr_form(const Launch &L, const TrArgs<T> &a) {
   if (use_quad(L, a.N)) return kFormQuad;
-  if constexpr (sizeof(T) == 4)
-    if (both_block(L, a)) return kFormBoth;
+  if (both_block(L, a)) return kFormBoth;
   return kFormOneLane;
 }
 int tr_eval_form(const Launch &L, const TrLayout &lay) {
   return lay.bw == 32 ? tr_form<uint32_t>(L, tr_args<uint32_t>(lay)) : tr_form<uint64_t>(L, tr_args<uint64_t>(lay));
+}
+
+template <typename T, int NT, int REP, int W>
+static void tr_both_launch(const Launch &L, const TrArgs<T> &a, const TrPool<T> *q) {
+  const int block = both_block(L, a);
+  const int grid = q ? grid_for(k_tr_eval_pool_b<T, NT, REP, W, 0>, block, a.N, L.num_cu)
+                     : grid_for(k_tr_eval_b<T, NT, REP, W, 0>, block, a.N, L.num_cu);
+  if (q && L.profiled)
+    hipLaunchKernelGGL((k_tr_eval_pool_b<T, NT, REP, W, 1>), dim3(grid), dim3(block), 0, L.stream, a, *q);
+  else if (q)
+    hipLaunchKernelGGL((k_tr_eval_pool_b<T, NT, REP, W, 0>), dim3(grid), dim3(block), 0, L.stream, a, *q);
+  else if (L.profiled)
+    hipLaunchKernelGGL((k_tr_eval_b<T, NT, REP, W, 1>), dim3(grid), dim3(block), 0, L.stream, a);
+  else
+    hipLaunchKernelGGL((k_tr_eval_b<T, NT, REP, W, 0>), dim3(grid), dim3(block), 0, L.stream, a);
 }
 
 // One gate evaluation of both parties with prepared arguments: the regular
@@ -839,13 +875,11 @@ static hipError_t tr_eval_launch(const Launch &L, const TrArgs<T> &a, const TrPo
   return with_variant(L, [&](auto v) {
     constexpr int NT = decltype(v)::nt, REP = decltype(v)::rep;
     if constexpr (sizeof(T) == 4) {
-      const int block = !q && tr_form(L, a) == kFormBoth ? both_block(L, a) : 0;
-      if (block) {
-        const int grid = grid_for(k_tr_eval_b<T, NT, REP, 0>, block, a.N, L.num_cu);
-        if (L.profiled)
-          hipLaunchKernelGGL((k_tr_eval_b<T, NT, REP, 1>), dim3(grid), dim3(block), 0, L.stream, a);
+      if (tr_form(L, a) == kFormBoth) {
+        if (both_waves(L, a) == 8)
+          tr_both_launch<T, NT, REP, 8>(L, a, q);
         else
-          hipLaunchKernelGGL((k_tr_eval_b<T, NT, REP, 0>), dim3(grid), dim3(block), 0, L.stream, a);
+          tr_both_launch<T, NT, REP, 4>(L, a, q);
         return hipGetLastError();
       }
     }
@@ -972,11 +1006,11 @@ hipError_t launch_tr_eval2(const Launch &L, const TrLayout &lay, const TrLayout 
     if constexpr (sizeof(T) == 4) {
       const int bb = both_block(L, a) ? both_block(L, a2) : 0;
       if (bb) {
-        const int grid = grid_for(k_tr_eval2_b<T, NT, REP, 0>, bb, lay.N, L.num_cu);
+        const int grid = grid_for(k_tr_eval2_b<T, NT, REP, 4, 0>, bb, lay.N, L.num_cu);
         if (L.profiled)
-          hipLaunchKernelGGL((k_tr_eval2_b<T, NT, REP, 1>), dim3(grid), dim3(bb), 0, L.stream, a, a2);
+          hipLaunchKernelGGL((k_tr_eval2_b<T, NT, REP, 4, 1>), dim3(grid), dim3(bb), 0, L.stream, a, a2);
         else
-          hipLaunchKernelGGL((k_tr_eval2_b<T, NT, REP, 0>), dim3(grid), dim3(bb), 0, L.stream, a, a2);
+          hipLaunchKernelGGL((k_tr_eval2_b<T, NT, REP, 4, 0>), dim3(grid), dim3(bb), 0, L.stream, a, a2);
         return hipGetLastError();
       }
     }

@@ -15,7 +15,7 @@
 
 namespace mpcx {
 
-constexpr int kBothAesAlone = 6, kBothAesLanes = 14;
+constexpr int kBothAesAlone = 64, kBothAesLanes = 14;
 constexpr int kBothMinAlone = 1024, kBothMinLanes = 512;
 struct Launch {
   hipStream_t stream = nullptr;
@@ -28,13 +28,15 @@ struct Launch {
   bool spread_small = true;
   // Longest gate (AES calls per element and party) whose launches of at least
   // both_min elements per CU run in the both-party form over Z_2^32: one thread
-  // per element holds both parties' keys (0 = never).  Gates of up to 6 calls
-  // gain alone and beside other streams' work; up to 14 only beside other
-  // streams' work (a model's lanes), and lose alone.  Alone a launch needs 1024
-  // elements per CU to give every CU a 1024-thread workgroup; beside other
-  // lanes' work 512 measured best (they fill the CUs it leaves).
+  // per element holds both parties' keys (0 = never; every gate by default).
+  // Alone a launch needs 1024 elements per CU to give every CU a 1024-thread
+  // workgroup (25-call gates: 150 against 155 us there, but 150 against 116 at
+  // 768); beside other lanes' work 512 measured best (they fill the CUs it leaves).
   int both_aes = kBothAesAlone;
   int both_min = kBothMinAlone;
+  // Other streams' launches run beside this one's: a both-party launch then
+  // leaves half of a CU's wave slots and LDS to them (both_waves).
+  bool shared = false;
   // Launches of a profiled forward use a separately named instantiation of the
   // DCF-evaluation kernel (same code), so kernel traces can tell them apart.
   bool profiled = false;

@@ -161,20 +161,18 @@ __global__ void k_dcf_eval(DcfEvalArgs<X> a) {
   AesLds<NT, REP>::fill(lds);
   AesLds<NT, REP> aes(lds);
   const size_t stride = size_t(gridDim.x) * blockDim.x;
-  const uint4 *root = reinterpret_cast<const uint4 *>(a.key + a.off_root);
-  const uint4 *cw = reinterpret_cast<const uint4 *>(a.key + a.off_cw);
-  const uint4 *leaf = reinterpret_cast<const uint4 *>(a.key + a.off_leaf);
-  const uint64_t *zp = reinterpret_cast<const uint64_t *>(a.key + a.off_z);
-  for (size_t base = size_t(blockIdx.x) * blockDim.x + (threadIdx.x & ~63u); base < a.n; base += stride) {
-    const size_t i = base + lane_id();
+  for (size_t base = size_t(blockIdx.x) * blockDim.x; base < a.n; base += stride) {
+    const size_t i = base + threadIdx.x;
     uint32_t b = 0;
     if (i < a.n) {
-      b = dcf_eval_walk(aes, root[i], a.m, a.L, cw + i, a.n, leaf[i], uint64_t(a.x[i]) & a.xmask);
-      b ^= get_bit(zp, i);
+      const DcfTile k{a.key + a.off_cw + 16 * base, a.key + a.off_leaf + 16 * base, 16 * a.n};
+      b = dcf_eval_walk(aes, ld16(a.key + a.off_root + 16 * base, 16 * threadIdx.x), a.m, a.L, k, 16 * threadIdx.x,
+                        X(a.x[i] & X(a.xmask)));
+      b ^= get_bit(reinterpret_cast<const uint64_t *>(a.key + a.off_z), i);
       if (a.mask) b ^= (a.mask[i >> 5] >> (i & 31)) & 1u;
     }
     const uint64_t w = __ballot(b);
-    if (lane_id() == 0) a.out[base >> 6] = w;
+    if (lane_id() == 0 && i < a.n) a.out[i >> 6] = w;
   }
 }
 

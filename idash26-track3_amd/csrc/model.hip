@@ -1649,6 +1649,7 @@ class Model final : public ModelBase, KeySource {
     // and bw = 64 unchanged, against none).
     const bool few = B <= kFewLaneB;
     L_.spread_small = few;
+    L_.shared = !alone_;
     L_.quad_per_cu = alone_ ? std::max(quad_base_, L_.quad_alone) : quad_base_;
     const int N = d_.n_nodes, bw = bw_;
     const size_t BN = size_t(B) * N;
@@ -1908,7 +1909,8 @@ hipError_t LaneSet::set_lanes(int n, std::string *e) {
     Launch Li = L_;
     if (i > 0) TRY(hipStreamCreateWithFlags(&Li.stream, hipStreamNonBlocking));
     // concurrent lanes keep the GPU busy beside each other's gates: the
-    // both-party form pays for longer gates there
+    // both-party form pays for smaller launches there, and for gates longer
+    // than a caller's own limit
     if (n > 1 && Li.both_aes > 0) {
       Li.both_aes = std::max(Li.both_aes, kBothAesLanes);
       Li.both_min = kBothMinLanes;
@@ -2340,6 +2342,7 @@ static hipError_t adjnorm_eval_t(int bw, int s, int B, int N, int nmax, int lane
     const int Bi = adj_lane_B(B, nl, i);
     const size_t g0 = size_t(adj_lane_off(B, nl, i));
     Launch Li = L;
+    Li.shared = nl > 1;
     if (i > 0) {
       // Group i starts once group i-1 has enqueued its memory-bound gates before
       // the truncation (which also orders it after the caller's stream): its

@@ -116,7 +116,7 @@ int mpcx_aes_variant(const mpcx_ctx *ctx);
 /* Longest truncation/ReLU gate, in AES calls per element and party, whose
  * Z_2^32 launches of at least 1024 elements per CU run in the both-party form
  * (one thread per element holds both parties' keys; same keys and outputs):
- * 0..64, default 6; 0 keeps every gate on the one-lane-per-party kernel.  A
+ * 0..64, default 64 (every gate); 0 keeps every gate on the one-lane-per-party kernel.  A
  * model with more than one lane takes max(setting, 14) for its own launches
  * (0 stays 0), from 512 elements per CU.  Read by the gate calls of this context and by models created
  * after it.  No counterpart in the reference: a tuning setting of this
