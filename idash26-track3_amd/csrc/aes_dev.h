@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "mpcx_core.h"
 
@@ -373,6 +374,14 @@ struct AesPerm2 {
     rounds(r, rk);
     return enc_out(r, rk);
   }
+  __device__ __forceinline__ void enc2(uint4 u, uint4 v, const AesRK &rk, uint4 *eu, uint4 *ev) const {
+    Reads a, b;
+    start(a, whiten(u, rk));
+    start(b, whiten(v, rk));
+    rounds2(a, rk, b, rk);
+    *eu = enc_out(a, rk);
+    *ev = enc_out(b, rk);
+  }
   __device__ __forceinline__ uint4 hash(uint4 s, const AesRK &rk) const {
     Reads r;
     start(r, hash_in(s, rk));
@@ -482,6 +491,19 @@ struct AesSel<2, 32> {
 };
 template <int NT, int REP>
 using AesLds = typename AesSel<NT, REP>::type;
+
+// Two dealer PRF blocks of one key and index, fields f0 and f1.
+template <class A>
+__device__ __forceinline__ void prf2(const A &aes, const AesRK &k, uint32_t gate, uint32_t f0, uint32_t f1,
+                                     uint64_t idx, uint4 *o0, uint4 *o1) {
+  if constexpr (std::is_same<A, AesPerm2>::value) {
+    const uint32_t lo = uint32_t(idx), hi = uint32_t(idx >> 32);
+    aes.enc2(make_uint4(lo, hi, f0, gate), make_uint4(lo, hi, f1, gate), k, o0, o1);
+  } else {
+    *o0 = aes.prf(k, gate, f0, idx);
+    *o1 = aes.prf(k, gate, f1, idx);
+  }
+}
 
 // a ^ (b & m) in one v_bitop3_b32 (truth table 0x78 = 0xf0 ^ (0xcc & 0xaa))
 __device__ __forceinline__ uint32_t xor_and(uint32_t a, uint32_t b, uint32_t m) {

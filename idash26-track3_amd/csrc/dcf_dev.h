@@ -153,65 +153,72 @@ __device__ __forceinline__ uint32_t dcf_eval_walk_quad(const AesQuad &aes, const
 
 struct DcfGenOut {
   uint4 s0;      // party 0's final on-path seed
-  uint32_t t0;   // party 0's final on-path control bit
+  uint32_t t0;   // party 0's final on-path control bit, as a mask
   uint4 leafcw;  // leaf correction word
 };
 
-// Dealer walk for one element from the parties' root seeds s0 (lsb 0) and s1
-// (lsb 1): writes the roots, the level correction words (level-major, stride N)
-// and the leaf correction word of both parties.
-template <class A>
-__device__ __forceinline__ DcfGenOut dcf_gen_roots(const A &aes, uint4 s0, uint4 s1, int m, int L, uint64_t alpha,
-                                                   size_t i, size_t N, uint8_t *k0, uint8_t *k1, size_t off_root,
-                                                   size_t off_cw, size_t off_leaf) {
+__device__ __forceinline__ void st16(uint8_t *base, uint32_t off, uint4 v) {
+  *reinterpret_cast<uint4 *>(base + off) = v;
+}
+// a ^ (b & ~m) in one v_bitop3_b32
+__device__ __forceinline__ uint32_t xor_not_and(uint32_t a, uint32_t b, uint32_t m) {
+  return __builtin_amdgcn_bitop3_b32(a, b, m, 0xb4);
+}
+
+// Dealer walk for element base + e from the parties' root seeds s0 (lsb 0) and s1
+// (lsb 1), both parties' seeds hashed side by side: writes the roots, the level
+// correction words (level-major) and the leaf correction word of both keys.
+// base is uniform over the wave.
+template <class A, typename X>
+__device__ __forceinline__ DcfGenOut dcf_gen_walk(const A &aes, uint4 s0, uint4 s1, const DcfLayout &d, X alpha,
+                                                  size_t base, uint32_t e, uint8_t *k0, uint8_t *k1) {
   const uint4 D = xor4(s0, s1);
-  reinterpret_cast<uint4 *>(k0 + off_root)[i] = s0;
-  reinterpret_cast<uint4 *>(k1 + off_root)[i] = s1;
-  uint32_t t0 = 0, t1 = 1;
-  uint4 *c0 = reinterpret_cast<uint4 *>(k0 + off_cw) + i;
-  uint4 *c1 = reinterpret_cast<uint4 *>(k1 + off_cw) + i;
-  for (int l = 0; l < L; l++) {
-    const uint32_t a = uint32_t(alpha >> (m - 1 - l)) & 1u;
-    const uint4 h0 = aes.hash(s0, c_rkH);
-    const uint4 h1 = aes.hash(s1, c_rkH);
-    const uint4 cw = xor4(xor4(h0, h1), and4(D, a - 1u));  // a ? 0 : D
-    c0[size_t(l) * N] = cw;
-    c1[size_t(l) * N] = cw;
-    const uint4 sl0 = xor4(h0, and4(cw, 0u - t0));
-    const uint4 sl1 = xor4(h1, and4(cw, 0u - t1));
-    s0 = xor4(sl0, and4(s0, 0u - a));
-    s1 = xor4(sl1, and4(s1, 0u - a));
-    t0 = s0.x & 1u;
-    t1 = s1.x & 1u;
+  const uint32_t off = 16 * e;
+  st16(k0 + d.off_root + 16 * base, off, s0);
+  st16(k1 + d.off_root + 16 * base, off, s1);
+  uint32_t t0 = 0, t1 = ~0u;
+  uint8_t *c0 = k0 + d.off_cw + 16 * base, *c1 = k1 + d.off_cw + 16 * base;
+  PathBits<X> path(alpha, d.m);
+  for (int l = 0; l < d.L; l++, c0 += 16 * d.N, c1 += 16 * d.N) {
+    const uint32_t a = path.next();
+    uint4 h0, h1;
+    hash_pair(aes, s0, s1, c_rkH, &h0, &h1);
+    uint4 cw;  // h0 ^ h1 ^ (a ? 0 : D)
+    cw.x = xor_not_and(h0.x ^ h1.x, D.x, a);
+    cw.y = xor_not_and(h0.y ^ h1.y, D.y, a);
+    cw.z = xor_not_and(h0.z ^ h1.z, D.z, a);
+    cw.w = xor_not_and(h0.w ^ h1.w, D.w, a);
+    st16(c0, off, cw);
+    st16(c1, off, cw);
+    s0 = xor_and4(xor_and4(h0, cw, t0), s0, a);
+    s1 = xor_and4(xor_and4(h1, cw, t1), s1, a);
+    t0 = bit_mask(s0.x, 0);
+    t1 = bit_mask(s1.x, 0);
   }
-  const uint32_t pos = m >= 7 ? uint32_t(alpha & 127u) : uint32_t(alpha);
-  uint4 lcw = xor4(aes.hash(s0, c_rkL), aes.hash(s1, c_rkL));
+  const uint32_t pos = path.leaf_pos(d.m);
+  uint4 l0, l1;
+  hash_pair(aes, s0, s1, c_rkL, &l0, &l1);
+  uint4 lcw = xor4(l0, l1);
   const uint32_t bitv = 1u << (pos & 31u);
   lcw.x ^= (pos >> 5) == 0 ? bitv : 0u;
   lcw.y ^= (pos >> 5) == 1 ? bitv : 0u;
   lcw.z ^= (pos >> 5) == 2 ? bitv : 0u;
   lcw.w ^= (pos >> 5) == 3 ? bitv : 0u;
-  reinterpret_cast<uint4 *>(k0 + off_leaf)[i] = lcw;
-  reinterpret_cast<uint4 *>(k1 + off_leaf)[i] = lcw;
-  DcfGenOut o;
-  o.s0 = s0;
-  o.t0 = t0;
-  o.leafcw = lcw;
-  return o;
+  st16(k0 + d.off_leaf + 16 * base, off, lcw);
+  st16(k1 + d.off_leaf + 16 * base, off, lcw);
+  return {s0, t0, lcw};
 }
 
-// The same with the roots drawn from the dealer PRF: s0 = PRF(fb) with lsb 0,
-// s1 = s0 ^ D, D = PRF(fb + 1) with lsb 1.
+// Roots drawn from the dealer PRF: s0 = PRF(fb) with lsb 0, s1 = s0 ^ D,
+// D = PRF(fb + 1) with lsb 1.
 template <class A>
-__device__ __forceinline__ DcfGenOut dcf_gen_walk(const A &aes, const AesRK &kd, uint32_t gate, uint32_t fb, int m, int L,
-                                                  uint64_t alpha, size_t i, size_t N, uint8_t *k0,
-                                                  uint8_t *k1, size_t off_root, size_t off_cw,
-                                                  size_t off_leaf) {
-  uint4 s0 = aes.prf(kd, gate, fb + 0, i);
-  s0.x &= ~1u;
-  uint4 D = aes.prf(kd, gate, fb + 1, i);
+__device__ __forceinline__ void dealer_roots(const A &aes, const AesRK &kd, uint32_t gate, uint32_t fb, size_t i,
+                                             uint4 *s0, uint4 *s1) {
+  uint4 D;
+  prf2(aes, kd, gate, fb, fb + 1, i, s0, &D);
+  s0->x &= ~1u;
   D.x |= 1u;
-  return dcf_gen_roots(aes, s0, xor4(s0, D), m, L, alpha, i, N, k0, k1, off_root, off_cw, off_leaf);
+  *s1 = xor4(*s0, D);
 }
 
 // Root seed of party p for a DCF drawn from the party's own PRF key: lsb = p.
@@ -220,6 +227,16 @@ __device__ __forceinline__ uint4 party_root(const A &aes, const AesRK &kp, int p
                                             size_t i) {
   uint4 s = aes.prf(kp, gate, fb + 0, i);
   s.x = (s.x & ~1u) | uint32_t(p);
+  return s;
+}
+// The same and the party's output-mask bit (field fb + 2).
+template <class A>
+__device__ __forceinline__ uint4 party_root_bit(const A &aes, const AesRK &kp, int p, uint32_t gate, uint32_t fb,
+                                                size_t i, uint32_t *z) {
+  uint4 s, b;
+  prf2(aes, kp, gate, fb, fb + 2, i, &s, &b);
+  s.x = (s.x & ~1u) | uint32_t(p);
+  *z = b.x & 1u;
   return s;
 }
 

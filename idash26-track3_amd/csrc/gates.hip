@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstddef>
 #include <type_traits>
 
 #include "dcf_dev.h"
@@ -26,8 +27,6 @@ namespace mpcx {
 // ---------------------------------------------------------------------------
 template <typename T>
 struct TrArgs {
-  AesRK kd;
-  AesRK kp[2];  // the parties' own PRF keys (keygen and seeded-plane expansion)
   int kind, n, s;
   int sb;        // sign bit of the shifted input (tr_sign_bit)
   int m, sh;     // input width (tr_in_bits) and the gate's own shift (tr_shift)
@@ -607,102 +606,165 @@ __global__ void k_tr_party_msg(TrArgs<T> a, int p, const uint64_t *own, const ui
   }
 }
 
-template <typename T, int NT, int REP>
-__global__ void k_tr_keygen(TrArgs<T> a) {
-  __shared__ __align__(16) uint32_t lds[AesLds<NT, REP>::kWords];
-  AesLds<NT, REP>::fill(lds);
-  AesLds<NT, REP> aes(lds);
-  const size_t stride = size_t(gridDim.x) * blockDim.x;
-  const int n = a.n, s = a.s;
-  const T lowmask = (T(1) << a.sb) - T(1);
-  const T smask = (T(1) << s) - T(1);
+// ---- dealer ----
+// The dealer's PRF key and the parties' own (every purely random plane of a
+// party's key comes from its own).
+struct TrKeys {
+  AesRK kd, kp[2];
+};
+// One launch's gates: `one` alone (ng = 0), or `many` of them, `tile0` the first
+// 64-element tile of each in the launch (tile0[ng] the number of tiles).
+template <typename T>
+struct TrGen {
+  TrArgs<T> a;
+  size_t tile0 = 0;
+  int has_rout = 0;  // the output mask is there already (its PRF block was drawn ahead)
+};
+template <typename T>
+struct TrGenArgs {
+  TrKeys keys;
+  TrGen<T> one;
+  const TrGen<T> *many = nullptr;
+  int ng = 0;
+  size_t tiles = 0;
+};
+
+// A value in uniform, unwritten memory (kernel arguments, a table of gates), read
+// into scalar registers.  fresh() hides where a pointer comes from, so that what
+// is read through it is read there: round keys of three keys at once would not
+// fit the scalar registers and be spilled to vector lanes.
+using ConstWord = const __attribute__((address_space(4))) uint32_t;
+template <class S>
+__device__ __forceinline__ S load_uniform(ConstWord *p) {
+  uint32_t w[sizeof(S) / 4];
+#pragma unroll
+  for (size_t k = 0; k < sizeof(S) / 4; k++) w[k] = p[k];
+  S s;
+  __builtin_memcpy(&s, w, sizeof(S));
+  return s;
+}
+__device__ __forceinline__ ConstWord *fresh(ConstWord *p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+// The dealer's entry c of a gate's G table before it is split: r the input mask,
+// rho its sign bit, rout the output mask, ba and bd the DCF output masks.
+template <typename T>
+__device__ __forceinline__ T tr_g_value(const TrArgs<T> &a, uint32_t c, T r, uint32_t rho, T rout, uint32_t ba,
+                                        uint32_t bd) {
+  const T R = r >> a.sh;
   const int wsh = a.m - a.sh;  // weight of the wrap bit after the shift
-  T *G0 = reinterpret_cast<T *>(a.w0 + a.off_g);
-  T *G1 = reinterpret_cast<T *>(a.w1 + a.off_g);
-  const int ncase = a.ncase;
-  for (size_t base = size_t(blockIdx.x) * blockDim.x + (threadIdx.x & ~63u); base < a.N; base += stride) {
-    const size_t i = base + lane_id();
-    uint32_t za0 = 0, za1 = 0, zb0 = 0, zb1 = 0;
-    if (i < a.N) {
-      const T r = low_bits<T>(a.in_mask[i], a.m);
-      const uint32_t rho = uint32_t(r >> a.sb) & 1u;
-      const T R = r >> a.sh;
-      // each party's output-mask bit of a DCF comes from its own PRF key; the
-      // DCF output mask is their XOR
-      if (a.use_a) {
-        za0 = aes.prf(a.kp[0], a.gate, F_DCFA + 2, i).x & 1u;
-        za1 = aes.prf(a.kp[1], a.gate, F_DCFA + 2, i).x & 1u;
-      }
-      if (a.use_b) {
-        zb0 = aes.prf(a.kp[0], a.gate, F_DCFB + 2, i).x & 1u;
-        zb1 = aes.prf(a.kp[1], a.gate, F_DCFB + 2, i).x & 1u;
-      }
-      const uint32_t rbi = za0 ^ za1, rdi = zb0 ^ zb1;
-      const T rout = ring_of<T>(aes.prf(a.kd, a.gate, F_ROUT, i));
-      const uint32_t kappa = rho ^ rbi;
-      a.out_mask[i] = a.kind == G_DRELU ? T(kappa) : rout;  // DRELU: the mask of the output bit
-      for (int c = 0; c < ncase; c++) {
-        T Gv;
-        if (a.kind == G_TRMOD) {
-          Gv = rout - R - T(uint32_t(c) ^ rdi);
-        } else if (a.kind == G_EXT || a.kind == G_EXTRELU) {
-          const uint32_t h = uint32_t(c) >> 1, b = (uint32_t(c) & 1u) ^ rbi;
-          const uint32_t w = h ? (rho & b) : (rho | b);
-          if (a.kind == G_EXTRELU) {
-            const T cc = T(h ^ rho ^ b);
-            Gv = rout - cc * R + ((cc * T(w)) << wsh);
-          } else {
-            Gv = rout - R + (T(w) << wsh);
-          }
-        } else if (a.kind == G_TR || a.kind == G_TRRELU) {
-          const uint32_t h = uint32_t(c) >> 2, bh = (uint32_t(c) >> 1) & 1u, dh = uint32_t(c) & 1u;
-          const uint32_t b = bh ^ rbi, d = dh ^ rdi;
-          const uint32_t w = h ? (rho & b) : (rho | b);
-          if (a.kind == G_TRRELU) {
-            const T cc = T(h ^ rho ^ b);
-            Gv = rout - cc * R - cc * T(d) + ((cc * T(w)) << (n - s));
-          } else {
-            Gv = rout - R - T(d) + (T(w) << (n - s));
-          }
-        } else if (relu_like(a.kind)) {
-          const T cc = T(uint32_t(c) ^ kappa);
-          Gv = rout - cc * r;
-        } else {
-          const uint32_t Hh = uint32_t(c) >> 1, dh = uint32_t(c) & 1u;
-          const uint32_t d = dh ^ rdi;
-          const uint32_t R2 = uint32_t(r >> (n - 2)) & 3u;
-          const uint32_t w = Hh < R2 ? 1u : 0u;
-          Gv = rout - R - T(d) + (T(w) << (n - s));
-        }
-        const T g0 = ring_of<T>(aes.prf(a.kp[0], a.gate, F_SPLIT + uint32_t(c), i));
-        G0[size_t(c) * a.N + i] = g0;
-        G1[size_t(c) * a.N + i] = Gv - g0;
+  if (a.kind == G_TRMOD) return rout - R - T(c ^ bd);
+  if (a.kind == G_EXT || a.kind == G_EXTRELU) {
+    const uint32_t h = c >> 1, b = (c & 1u) ^ ba, w = h ? (rho & b) : (rho | b);
+    if (a.kind == G_EXT) return rout - R + (T(w) << wsh);
+    const T cc = T(h ^ rho ^ b);
+    return rout - cc * R + ((cc * T(w)) << wsh);
+  }
+  if (a.kind == G_TR || a.kind == G_TRRELU) {
+    const uint32_t h = c >> 2, b = ((c >> 1) & 1u) ^ ba, d = (c & 1u) ^ bd, w = h ? (rho & b) : (rho | b);
+    if (a.kind == G_TR) return rout - R - T(d) + (T(w) << (a.n - a.s));
+    const T cc = T(h ^ rho ^ b);
+    return rout - cc * R - cc * T(d) + ((cc * T(w)) << (a.n - a.s));
+  }
+  if (relu_like(a.kind)) return rout - T(c ^ rho ^ ba) * r;
+  // G_TRSLACK
+  const uint32_t R2 = uint32_t(r >> (a.n - 2)) & 3u, w = (c >> 1) < R2 ? 1u : 0u;
+  return rout - R - T((c & 1u) ^ bd) + (T(w) << (a.n - a.s));
+}
+
+// Both parties' keys of the 64 elements from base on of gate a.
+template <typename T, class Aes>
+__device__ __forceinline__ void tr_gen_tile(const Aes &aes, ConstWord *keys, const TrGen<T> &g, size_t base) {
+  constexpr int kWords = sizeof(AesRK) / 4;
+  const TrArgs<T> &a = g.a;
+  const uint32_t e = lane_id();
+  const size_t i = base + e;
+  const bool in = i < a.N;
+  uint32_t za0 = 0, za1 = 0, zb0 = 0, zb1 = 0;
+  if (in) {
+    const T r = low_bits<T>(a.in_mask[i], a.m);
+    const uint32_t rho = uint32_t(r >> a.sb) & 1u;
+    uint4 ra0, ra1, rb0, rb1;
+    {  // each party's roots and output-mask bits come from its own key
+      const AesRK k = load_uniform<AesRK>(fresh(keys + 2 * kWords));
+      if (a.use_a) ra1 = party_root_bit(aes, k, 1, a.gate, F_DCFA, i, &za1);
+      if (a.use_b) rb1 = party_root_bit(aes, k, 1, a.gate, F_DCFB, i, &zb1);
+    }
+    T rout;
+    if (g.has_rout)
+      rout = a.out_mask[i];
+    else
+      rout = ring_of<T>(aes.prf(load_uniform<AesRK>(fresh(keys)), a.gate, F_ROUT, i));
+    {
+      const AesRK k = load_uniform<AesRK>(fresh(keys + kWords));
+      if (a.use_a) ra0 = party_root_bit(aes, k, 0, a.gate, F_DCFA, i, &za0);
+      if (a.use_b) rb0 = party_root_bit(aes, k, 0, a.gate, F_DCFB, i, &zb0);
+      const uint32_t ba = za0 ^ za1, bd = zb0 ^ zb1, kappa = rho ^ ba;
+      // DRELU: the output mask is the mask of the output bit
+      if (!g.has_rout) a.out_mask[i] = a.kind == G_DRELU ? T(kappa) : rout;
+      T *G0 = reinterpret_cast<T *>(a.w0 + a.off_g), *G1 = reinterpret_cast<T *>(a.w1 + a.off_g);
+      for (int c = 0; c < a.ncase; c += 2) {  // 0, 2, 4 or 8 entries
+        uint4 p, q;
+        prf2(aes, k, a.gate, F_SPLIT + uint32_t(c), F_SPLIT + uint32_t(c) + 1, i, &p, &q);
+        const T p0 = ring_of<T>(p), q0 = ring_of<T>(q);
+        G0[size_t(c) * a.N + i] = p0;
+        G1[size_t(c) * a.N + i] = tr_g_value(a, uint32_t(c), r, rho, rout, ba, bd) - p0;
+        G0[size_t(c + 1) * a.N + i] = q0;
+        G1[size_t(c + 1) * a.N + i] = tr_g_value(a, uint32_t(c) + 1, r, rho, rout, ba, bd) - q0;
       }
       if (a.relu) {
-        const T q0 = ring_of<T>(aes.prf(a.kp[0], a.gate, F_SPLIT + 8, i));
+        const T q0 = ring_of<T>(aes.prf(k, a.gate, F_SPLIT + 8, i));
         reinterpret_cast<T *>(a.w0 + a.off_kappa)[i] = q0;
         reinterpret_cast<T *>(a.w1 + a.off_kappa)[i] = T(kappa) - q0;
       }
-      if (a.use_a)
-        dcf_gen_roots(aes, party_root(aes, a.kp[0], 0, a.gate, F_DCFA, i),
-                      party_root(aes, a.kp[1], 1, a.gate, F_DCFA, i), a.a.m, a.a.L, uint64_t(r & lowmask), i, a.N,
-                      a.w0, a.w1, a.a.off_root, a.a.off_cw, a.a.off_leaf);
-      if (a.use_b)
-        dcf_gen_roots(aes, party_root(aes, a.kp[0], 0, a.gate, F_DCFB, i),
-                      party_root(aes, a.kp[1], 1, a.gate, F_DCFB, i), a.b.m, a.b.L, uint64_t(r & smask), i, a.N,
-                      a.w0, a.w1, a.b.off_root, a.b.off_cw, a.b.off_leaf);
     }
-    const uint64_t wa0 = __ballot(za0), wa1 = __ballot(za1), wb0 = __ballot(zb0), wb1 = __ballot(zb1);
-    if (lane_id() == 0) {
-      if (a.use_a) {
-        reinterpret_cast<uint64_t *>(a.w0 + a.a.off_z)[base >> 6] = wa0;
-        reinterpret_cast<uint64_t *>(a.w1 + a.a.off_z)[base >> 6] = wa1;
-      }
-      if (a.use_b) {
-        reinterpret_cast<uint64_t *>(a.w0 + a.b.off_z)[base >> 6] = wb0;
-        reinterpret_cast<uint64_t *>(a.w1 + a.b.off_z)[base >> 6] = wb1;
+    const T lowmask = (T(1) << a.sb) - T(1), smask = (T(1) << a.s) - T(1);
+    if (a.use_a) dcf_gen_walk(aes, ra0, ra1, a.a, T(r & lowmask), base, e, a.w0, a.w1);
+    if (a.use_b) dcf_gen_walk(aes, rb0, rb1, a.b, T(r & smask), base, e, a.w0, a.w1);
+  }
+  const uint64_t wa0 = __ballot(za0), wa1 = __ballot(za1), wb0 = __ballot(zb0), wb1 = __ballot(zb1);
+  if (e == 0) {
+    if (a.use_a) {
+      reinterpret_cast<uint64_t *>(a.w0 + a.a.off_z)[base >> 6] = wa0;
+      reinterpret_cast<uint64_t *>(a.w1 + a.a.off_z)[base >> 6] = wa1;
+    }
+    if (a.use_b) {
+      reinterpret_cast<uint64_t *>(a.w0 + a.b.off_z)[base >> 6] = wb0;
+      reinterpret_cast<uint64_t *>(a.w1 + a.b.off_z)[base >> 6] = wb1;
+    }
+  }
+}
+
+// The tiles of a launch's gates, dealt to the workgroups in turn, wave by wave.
+// Bound by the table reads (5634 per element of an EXTRELU gate: the two walks
+// 4160, the PRF blocks the rest) and, for few elements, by the chain of blocks a
+// thread runs one after another: each pair of PRF blocks of one key and the two
+// parties' hashes of a level run as two chains, which halves that chain and keeps
+// 32 reads in flight.  1.4 M EXTRELU elements 620 -> 535 us, 262144 132 -> 105,
+// 1024 74 -> 42 (one block at a time, and 112 registers spilled, before).
+template <typename T, int NT, int REP>
+__global__ void __launch_bounds__(1024, 4) k_tr_keygen(TrGenArgs<T> ka) {
+  __shared__ __align__(16) uint32_t lds[AesLds<NT, REP>::kWords];
+  AesLds<NT, REP>::fill(lds);
+  const AesLds<NT, REP> aes(lds);
+  ConstWord *args = (ConstWord *)__builtin_amdgcn_kernarg_segment_ptr();
+  const size_t wave = size_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  const size_t stride = size_t(gridDim.x) * (blockDim.x >> 6);
+  for (size_t t = wave * gridDim.x + blockIdx.x; t < ka.tiles; t += stride) {
+    ConstWord *at = args + offsetof(TrGenArgs<T>, one) / 4;
+    if (ka.ng) {
+      at = (ConstWord *)(uintptr_t)ka.many;
+      constexpr int kStep = int(sizeof(TrGen<T>) / 4);
+      for (int k = 1; k < ka.ng; k++) {  // the last gate that starts at or before t
+        ConstWord *n = at + kStep;
+        if (load_uniform<size_t>(n + offsetof(TrGen<T>, tile0) / 4) > t) break;
+        at = n;
       }
     }
+    const TrGen<T> g = load_uniform<TrGen<T>>(fresh(at));
+    tr_gen_tile<T>(aes, args + offsetof(TrGenArgs<T>, keys) / 4, g, 64 * (t - g.tile0));
   }
 }
 
@@ -729,26 +791,43 @@ static TrArgs<T> tr_args(const TrLayout &lay) {
   return a;
 }
 
+// One launch over ka.tiles tiles.  Few tiles go to 256-thread workgroups, whose
+// waves are spread over the CUs before a workgroup takes a second one.
 template <typename T>
-hipError_t launch_tr_keygen(const Launch &L, const TrLayout &lay, uint64_t seed, uint32_t gate, const T *in_mask,
-                            T *out_mask, uint8_t *k0, uint8_t *k1) {
-  if (lay.bw != int(8 * sizeof(T))) return hipErrorInvalidValue;
+static hipError_t tr_gen_launch(const Launch &L, const TrGenArgs<T> &ka) {
+  return with_variant(L, [&](auto v) {
+    constexpr int NT = decltype(v)::nt, REP = decltype(v)::rep;
+    const int block = L.aes_block > 0 ? L.aes_block : ka.tiles < 8 * size_t(L.num_cu) ? 256 : 1024;
+    const int occ_grid = grid_for(k_tr_keygen<T, NT, REP>, block, size_t(-1) / 2, L.num_cu);
+    const int grid = int(std::min<size_t>(size_t(occ_grid), ka.tiles));
+    hipLaunchKernelGGL((k_tr_keygen<T, NT, REP>), dim3(grid), dim3(block), 0, L.stream, ka);
+    return hipGetLastError();
+  });
+}
+static TrKeys tr_keys(const Launch &L, uint64_t seed) {
+  return {dealer_key(L, seed), {party_key(L, seed, 0), party_key(L, seed, 1)}};
+}
+template <typename T>
+static TrArgs<T> tr_gen_args(const TrLayout &lay, uint32_t gate, const T *in_mask, T *out_mask, uint8_t *k0,
+                             uint8_t *k1) {
   TrArgs<T> a = tr_args<T>(lay);
-  a.kd = dealer_key(L, seed);
-  a.kp[0] = party_key(L, seed, 0);
-  a.kp[1] = party_key(L, seed, 1);
   a.gate = gate;
   a.w0 = k0;
   a.w1 = k1;
   a.in_mask = in_mask;
   a.out_mask = out_mask;
-  return with_variant(L, [&](auto v) {
-    constexpr int NT = decltype(v)::nt, REP = decltype(v)::rep;
-    int block = variant_block(L);
-    int grid = grid_for(k_tr_keygen<T, NT, REP>, block, lay.N, L.num_cu);
-    hipLaunchKernelGGL((k_tr_keygen<T, NT, REP>), dim3(grid), dim3(block), 0, L.stream, a);
-    return hipGetLastError();
-  });
+  return a;
+}
+
+template <typename T>
+hipError_t launch_tr_keygen(const Launch &L, const TrLayout &lay, uint64_t seed, uint32_t gate, const T *in_mask,
+                            T *out_mask, uint8_t *k0, uint8_t *k1) {
+  if (lay.bw != int(8 * sizeof(T))) return hipErrorInvalidValue;
+  TrGenArgs<T> ka;
+  ka.keys = tr_keys(L, seed);
+  ka.one.a = tr_gen_args(lay, gate, in_mask, out_mask, k0, k1);
+  ka.tiles = (lay.N + 63) / 64;
+  return tr_gen_launch(L, ka);
 }
 
 // A gate evaluation of fewer elements than this is latency-bound (a few
@@ -1065,11 +1144,10 @@ hipError_t launch_tr_party_msg(const Launch &L, const TrLayout &lay, const uint8
 }
 
 template <typename T, int NT, int REP>
-__global__ void k_tr_expand(TrArgs<T> a, int p) {
+__global__ void k_tr_expand(TrArgs<T> a, AesRK kp, int p) {
   __shared__ __align__(16) uint32_t lds[AesLds<NT, REP>::kWords];
   AesLds<NT, REP>::fill(lds);
   AesLds<NT, REP> aes(lds);
-  const AesRK &kp = a.kp[0];
   uint8_t *w = a.w0;
   const size_t stride = size_t(gridDim.x) * blockDim.x;
   const int ncase = a.ncase;
@@ -1107,14 +1185,14 @@ hipError_t launch_tr_expand(const Launch &L, const TrLayout &lay, const uint8_t 
   if (lay.bw != int(8 * sizeof(T)) || (party != 0 && party != 1)) return hipErrorInvalidValue;
   if (lay.N == 0 || lay.kind == G_LOCALARS) return hipSuccess;
   TrArgs<T> a = tr_args<T>(lay);
-  a.kp[0] = aes_expand(party_key16);
+  const AesRK kp = aes_expand(party_key16);
   a.gate = gate;
   a.w0 = key;
   return with_variant(L, [&](auto v) {
     constexpr int NT = decltype(v)::nt, REP = decltype(v)::rep;
     int block = variant_block(L);
     int grid = grid_for(k_tr_expand<T, NT, REP>, block, lay.N, L.num_cu);
-    hipLaunchKernelGGL((k_tr_expand<T, NT, REP>), dim3(grid), dim3(block), 0, L.stream, a, party);
+    hipLaunchKernelGGL((k_tr_expand<T, NT, REP>), dim3(grid), dim3(block), 0, L.stream, a, kp, party);
     return hipGetLastError();
   });
 }

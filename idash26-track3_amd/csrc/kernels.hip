@@ -82,12 +82,11 @@ hipError_t launch_prf(const Launch &L, uint64_t seed, uint32_t gate, uint32_t fi
 struct DcfGenArgs {
   AesRK kd;
   uint32_t gate, fb;
-  int m, L;
   size_t n;
   const uint64_t *alpha;
   const uint8_t *rbit;
   uint8_t *k0, *k1;
-  size_t off_root, off_cw, off_leaf, off_z;
+  DcfLayout lay;
 };
 
 template <int NT, int REP>
@@ -96,19 +95,20 @@ __global__ void k_dcf_keygen(DcfGenArgs a) {
   AesLds<NT, REP>::fill(lds);
   AesLds<NT, REP> aes(lds);
   const size_t stride = size_t(gridDim.x) * blockDim.x;
-  for (size_t base = size_t(blockIdx.x) * blockDim.x + (threadIdx.x & ~63u); base < a.n; base += stride) {
-    const size_t i = base + lane_id();
+  for (size_t base = size_t(blockIdx.x) * blockDim.x; base < a.n; base += stride) {
+    const size_t i = base + threadIdx.x;
     uint32_t z0 = 0, z1 = 0;
     if (i < a.n) {
-      dcf_gen_walk(aes, a.kd, a.gate, a.fb, a.m, a.L, a.alpha[i], i, a.n, a.k0, a.k1, a.off_root,
-                   a.off_cw, a.off_leaf);
+      uint4 s0, s1;
+      dealer_roots(aes, a.kd, a.gate, a.fb, i, &s0, &s1);
+      dcf_gen_walk(aes, s0, s1, a.lay, a.alpha[i], base, threadIdx.x, a.k0, a.k1);
       z0 = aes.prf(a.kd, a.gate, a.fb + 2, i).x & 1u;
       z1 = z0 ^ (a.rbit ? (a.rbit[i] & 1u) : 0u);
     }
     const uint64_t w0 = __ballot(z0), w1 = __ballot(z1);
-    if (lane_id() == 0) {
-      reinterpret_cast<uint64_t *>(a.k0 + a.off_z)[base >> 6] = w0;
-      reinterpret_cast<uint64_t *>(a.k1 + a.off_z)[base >> 6] = w1;
+    if (lane_id() == 0 && i < a.n) {
+      reinterpret_cast<uint64_t *>(a.k0 + a.lay.off_z)[i >> 6] = w0;
+      reinterpret_cast<uint64_t *>(a.k1 + a.lay.off_z)[i >> 6] = w1;
     }
   }
 }
@@ -120,17 +120,12 @@ hipError_t launch_dcf_keygen(const Launch &L, uint64_t seed, uint32_t gate, uint
   a.kd = dealer_key(L, seed);
   a.gate = gate;
   a.fb = fbase;
-  a.m = m;
-  a.L = lay.L;
   a.n = n;
   a.alpha = alpha;
   a.rbit = rbit;
   a.k0 = k0;
   a.k1 = k1;
-  a.off_root = lay.off_root;
-  a.off_cw = lay.off_cw;
-  a.off_leaf = lay.off_leaf;
-  a.off_z = lay.off_z;
+  a.lay = lay;
   return with_variant(L, [&](auto v) {
     constexpr int NT = decltype(v)::nt, REP = decltype(v)::rep;
     int block = variant_block(L);
@@ -773,11 +768,14 @@ __global__ void k_lut8_keygen(AesRK kd, uint32_t gate, Lut8Layout lay, const T *
   AesLds<NT, REP>::fill(lds);
   AesLds<NT, REP> aes(lds);
   const size_t N = lay.dpf.N;
-  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < N; i += size_t(gridDim.x) * blockDim.x) {
-    const uint64_t alpha = uint64_t(in_mask[i]) & 255u;
-    const DcfGenOut g = dcf_gen_walk(aes, kd, gate, F_DCFA, 8, lay.dpf.L, alpha, i, N, k0, k1,
-                                     lay.dpf.off_root, lay.dpf.off_cw, lay.dpf.off_leaf);
-    const uint4 lb = xor4(aes.hash(g.s0, c_rkL), and4(g.leafcw, 0u - g.t0));
+  for (size_t base = size_t(blockIdx.x) * blockDim.x; base < N; base += size_t(gridDim.x) * blockDim.x) {
+    const size_t i = base + threadIdx.x;
+    if (i >= N) break;
+    const uint32_t alpha = uint32_t(in_mask[i]) & 255u;
+    uint4 root0, root1;
+    dealer_roots(aes, kd, gate, F_DCFA, i, &root0, &root1);
+    const DcfGenOut g = dcf_gen_walk(aes, root0, root1, lay.dpf, alpha, base, threadIdx.x, k0, k1);
+    const uint4 lb = xor4(aes.hash(g.s0, c_rkL), and4(g.leafcw, g.t0));
     const uint32_t pos = uint32_t(alpha & 127u);
     const uint32_t wsel = pos >> 5;
     const uint32_t word = wsel == 0 ? lb.x : wsel == 1 ? lb.y : wsel == 2 ? lb.z : lb.w;

@@ -65,3 +65,23 @@ def test_maxpool_form_edges(mp, num_cu, extra):
         assert np.array_equal(got, x.reshape(N, C).max(0))
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("bw,kind,extra", [(32, "EXTRELU", -1), (32, "EXTRELU", 65), (64, "TRMOD", 1),
+                                           (64, "TRRELU", -63), (32, "DRELU", 0)])
+def test_keygen_form_edges(mp, orc, num_cu, bw, kind, extra):
+    """The dealer at the line between its 256- and 1024-thread workgroups (512
+    elements per CU): both keys and the output mask as the oracle's dealer writes
+    them, byte for byte."""
+    n = 512 * num_cu + extra
+    c = mp.Ctx(bw=bw, scale=S)
+    try:
+        code = getattr(mp, kind)
+        rin = _inputs(n, bw, 1, 77 + extra)[1]
+        k0, k1, ro = c.tr_keygen(code, rin, seed=11, gate=4)
+        o0, o1, oro = orc.tr_keygen(11, 4, code, bw, S, rin)
+        assert np.array_equal(ro.astype(np.uint64), oro.astype(np.uint64))
+        for got, want in ((k0, o0), (k1, o1)):
+            assert np.array_equal(mp.from_dev(got, np.uint8), np.asarray(want, np.uint8).reshape(-1))
+    finally:
+        c.close()
