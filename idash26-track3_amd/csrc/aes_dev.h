@@ -492,17 +492,24 @@ struct AesSel<2, 32> {
 template <int NT, int REP>
 using AesLds = typename AesSel<NT, REP>::type;
 
-// Two dealer PRF blocks of one key and index, fields f0 and f1.
+// Two dealer PRF blocks of one key, side by side where the table type can.
+template <class A>
+__device__ __forceinline__ void enc_pair(const A &aes, const AesRK &k, uint4 u, uint4 v, uint4 *eu, uint4 *ev) {
+  if constexpr (std::is_same<A, AesPerm2>::value) {
+    aes.enc2(u, v, k, eu, ev);
+  } else {
+    *eu = aes.enc(u, k);
+    *ev = aes.enc(v, k);
+  }
+}
+__device__ __forceinline__ uint4 prf_block(uint32_t gate, uint32_t field, uint64_t idx) {
+  return make_uint4(uint32_t(idx), uint32_t(idx >> 32), field, gate);
+}
+// fields f0 and f1 of index idx
 template <class A>
 __device__ __forceinline__ void prf2(const A &aes, const AesRK &k, uint32_t gate, uint32_t f0, uint32_t f1,
                                      uint64_t idx, uint4 *o0, uint4 *o1) {
-  if constexpr (std::is_same<A, AesPerm2>::value) {
-    const uint32_t lo = uint32_t(idx), hi = uint32_t(idx >> 32);
-    aes.enc2(make_uint4(lo, hi, f0, gate), make_uint4(lo, hi, f1, gate), k, o0, o1);
-  } else {
-    *o0 = aes.prf(k, gate, f0, idx);
-    *o1 = aes.prf(k, gate, f1, idx);
-  }
+  enc_pair(aes, k, prf_block(gate, f0, idx), prf_block(gate, f1, idx), o0, o1);
 }
 
 // a ^ (b & m) in one v_bitop3_b32 (truth table 0x78 = 0xf0 ^ (0xcc & 0xaa))

@@ -553,22 +553,37 @@ static mpcx_status maxpool_keygen_t(mpcx_ctx *c, int B, int N, int C, const void
   TrLayout lay[kMaxPoolLevels];
   int pairs[kMaxPoolLevels];
   const int Lv = maxpool_plan(c, B, N, C, lay, pairs);
-  const size_t rows = size_t(B) * N * C, P0 = Lv ? size_t(B) * pairs[0] * C : 0;
+  const size_t rows = size_t(B) * N * C;
+  size_t np = 0;  // pairs of all levels
+  for (int l = 0; l < Lv; l++) np += lay[l].N;
   void *sp = nullptr;
-  HIPC(c, ctx_work(c, (2 * rows + 2 * P0) * sizeof(T), &sp), "hipMalloc");
-  T *va = static_cast<T *>(sp), *vb = va + rows, *dm = vb + rows, *ym = dm + P0;
+  HIPC(c, ctx_work(c, (2 * rows + 2 * np) * sizeof(T), &sp), "hipMalloc");
+  T *va = static_cast<T *>(sp), *vb = va + rows, *dm = vb + rows, *ym = dm + np;
   const T *cur = static_cast<const T *>(in_mask);
   T *nxt = va;
-  uint8_t *K0 = static_cast<uint8_t *>(k0), *K1 = static_cast<uint8_t *>(k1);
+  // every level's output masks are PRF blocks and come first; the levels' input
+  // masks follow from them, and then all keys are written together
+  TrGenItem<T> items[kMaxPoolLevels];
+  size_t o = 0;
+  for (int l = 0; l < Lv; l++) {
+    items[l].lay = lay[l];
+    items[l].gate = gate + uint32_t(l);
+    items[l].in = dm + o;
+    items[l].out = ym + o;
+    o += lay[l].N;
+  }
+  HIPC(c, launch_tr_masks<T>(c->L, seed, items, size_t(Lv)), "maxpool_keygen");
   int R = N;
   for (int l = 0; l < Lv; l++) {
-    HIPC(c, launch_pool_diff<T>(c->L, B, R, C, cur, dm), "maxpool_keygen");
-    HIPC(c, launch_tr_keygen<T>(c->L, lay[l], seed, gate + uint32_t(l), dm, ym, K0, K1), "maxpool_keygen");
-    HIPC(c, launch_pool_combine<T>(c->L, B, R, C, cur, ym, nullptr, nxt), "maxpool_keygen");
+    HIPC(c, launch_pool_masks<T>(c->L, B, R, C, cur, items[l].out, dm + (items[l].out - ym), nxt), "maxpool_keygen");
     cur = nxt;
     nxt = nxt == va ? vb : va;
     R = pairs[l] + (R & 1);
   }
+  HIPC(c,
+       launch_tr_keygen_batch<T>(c->L, seed, items, size_t(Lv), static_cast<uint8_t *>(k0),
+                                 static_cast<uint8_t *>(k1)),
+       "maxpool_keygen");
   HIPC(c, hipMemcpyAsync(out_mask, cur, size_t(B) * C * sizeof(T), hipMemcpyDeviceToDevice, c->L.stream),
        "maxpool_keygen");
   HIPC(c, hipStreamSynchronize(c->L.stream), "sync");

@@ -612,25 +612,24 @@ __global__ void k_tr_party_msg(TrArgs<T> a, int p, const uint64_t *own, const ui
 struct TrKeys {
   AesRK kd, kp[2];
 };
-// One launch's gates: `one` alone (ng = 0), or `many` of them, `tile0` the first
-// 64-element tile of each in the launch (tile0[ng] the number of tiles).
+// A launch's gates, `tile0` the first 64-element tile of each in the launch.
 template <typename T>
 struct TrGen {
   TrArgs<T> a;
   size_t tile0 = 0;
   int has_rout = 0;  // the output mask is there already (its PRF block was drawn ahead)
 };
+constexpr int kGenGates = 8;
 template <typename T>
 struct TrGenArgs {
   TrKeys keys;
-  TrGen<T> one;
-  const TrGen<T> *many = nullptr;
+  TrGen<T> g[kGenGates];
   int ng = 0;
   size_t tiles = 0;
 };
 
-// A value in uniform, unwritten memory (kernel arguments, a table of gates), read
-// into scalar registers.  fresh() hides where a pointer comes from, so that what
+// A value in uniform, unwritten memory (kernel arguments), read into scalar
+// registers.  fresh() hides where a pointer comes from, so that what
 // is read through it is read there: round keys of three keys at once would not
 // fit the scalar registers and be spilled to vector lanes.
 using ConstWord = const __attribute__((address_space(4))) uint32_t;
@@ -753,15 +752,12 @@ __global__ void __launch_bounds__(1024, 4) k_tr_keygen(TrGenArgs<T> ka) {
   const size_t wave = size_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
   const size_t stride = size_t(gridDim.x) * (blockDim.x >> 6);
   for (size_t t = wave * gridDim.x + blockIdx.x; t < ka.tiles; t += stride) {
-    ConstWord *at = args + offsetof(TrGenArgs<T>, one) / 4;
-    if (ka.ng) {
-      at = (ConstWord *)(uintptr_t)ka.many;
-      constexpr int kStep = int(sizeof(TrGen<T>) / 4);
-      for (int k = 1; k < ka.ng; k++) {  // the last gate that starts at or before t
-        ConstWord *n = at + kStep;
-        if (load_uniform<size_t>(n + offsetof(TrGen<T>, tile0) / 4) > t) break;
-        at = n;
-      }
+    static_assert(sizeof(TrGenArgs<T>) <= 4096, "kernel arguments");
+    ConstWord *at = args + offsetof(TrGenArgs<T>, g) / 4;
+    for (int k = 1; k < ka.ng; k++) {  // the last gate that starts at or before t
+      ConstWord *n = at + sizeof(TrGen<T>) / 4;
+      if (load_uniform<size_t>(n + offsetof(TrGen<T>, tile0) / 4) > t) break;
+      at = n;
     }
     const TrGen<T> g = load_uniform<TrGen<T>>(fresh(at));
     tr_gen_tile<T>(aes, args + offsetof(TrGenArgs<T>, keys) / 4, g, 64 * (t - g.tile0));
@@ -825,9 +821,102 @@ hipError_t launch_tr_keygen(const Launch &L, const TrLayout &lay, uint64_t seed,
   if (lay.bw != int(8 * sizeof(T))) return hipErrorInvalidValue;
   TrGenArgs<T> ka;
   ka.keys = tr_keys(L, seed);
-  ka.one.a = tr_gen_args(lay, gate, in_mask, out_mask, k0, k1);
+  ka.g[0].a = tr_gen_args(lay, gate, in_mask, out_mask, k0, k1);
+  ka.ng = 1;
   ka.tiles = (lay.N + 63) / 64;
   return tr_gen_launch(L, ka);
+}
+
+// Output masks of several gates: tiles of 128 elements, two PRF blocks a thread.
+constexpr int kMaskGates = 64;
+template <typename T>
+struct TrMaskArgs {
+  AesRK kd;
+  struct {
+    T *out;
+    size_t n, tile0;
+    uint32_t gate;
+  } g[kMaskGates];
+  int ng = 0;
+  size_t tiles = 0;
+};
+template <typename T, int NT, int REP>
+__global__ void __launch_bounds__(1024, 4) k_tr_masks(TrMaskArgs<T> a) {
+  __shared__ __align__(16) uint32_t lds[AesLds<NT, REP>::kWords];
+  AesLds<NT, REP>::fill(lds);
+  const AesLds<NT, REP> aes(lds);
+  const size_t wave = size_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  const size_t stride = size_t(gridDim.x) * (blockDim.x >> 6);
+  int k = 0;
+  for (size_t t = wave * gridDim.x + blockIdx.x; t < a.tiles; t += stride) {
+    while (k + 1 < a.ng && a.g[k + 1].tile0 <= t) k++;
+    const size_t i = 128 * (t - a.g[k].tile0) + lane_id(), j = i + 64;
+    uint4 p, q;
+    enc_pair(aes, a.kd, prf_block(a.g[k].gate, F_ROUT, i), prf_block(a.g[k].gate, F_ROUT, j), &p, &q);
+    if (i < a.g[k].n) a.g[k].out[i] = ring_of<T>(p);
+    if (j < a.g[k].n) a.g[k].out[j] = ring_of<T>(q);
+  }
+}
+template <typename T>
+hipError_t launch_tr_masks(const Launch &L, uint64_t seed, const TrGenItem<T> *items, size_t n) {
+  TrMaskArgs<T> a;
+  a.kd = dealer_key(L, seed);
+  for (size_t first = 0; first < n; first += kMaskGates) {
+    a.ng = int(std::min<size_t>(kMaskGates, n - first));
+    a.tiles = 0;
+    for (int k = 0; k < a.ng; k++) {
+      const TrGenItem<T> &it = items[first + size_t(k)];
+      a.g[k] = {it.out, it.lay.N, a.tiles, it.gate};
+      a.tiles += (it.lay.N + 127) / 128;
+    }
+    if (a.tiles == 0) continue;
+    const hipError_t e = with_variant(L, [&](auto v) {
+      constexpr int NT = decltype(v)::nt, REP = decltype(v)::rep;
+      const int block = L.aes_block > 0 ? L.aes_block : a.tiles < 8 * size_t(L.num_cu) ? 256 : 1024;
+      const int occ_grid = grid_for(k_tr_masks<T, NT, REP>, block, size_t(-1) / 2, L.num_cu);
+      const int grid = int(std::min<size_t>(size_t(occ_grid), a.tiles));
+      hipLaunchKernelGGL((k_tr_masks<T, NT, REP>), dim3(grid), dim3(block), 0, L.stream, a);
+      return hipGetLastError();
+    });
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+// The largest gates share launches, so that their long tails overlap; the small
+// ones, which alone would each cost their chain of some 20 blocks (42 us however
+// few elements), run together in the last.
+template <typename T>
+hipError_t launch_tr_keygen_batch(const Launch &L, uint64_t seed, const TrGenItem<T> *items, size_t n, uint8_t *k0,
+                                  uint8_t *k1) {
+  constexpr size_t kMost = 64;
+  const TrGenItem<T> *order[kMost];
+  size_t no = 0;
+  if (n > kMost) return hipErrorInvalidValue;
+  for (size_t k = 0; k < n; k++) {
+    if (items[k].lay.bw != int(8 * sizeof(T)) || items[k].lay.kind == G_DRELU) return hipErrorInvalidValue;
+    if (items[k].lay.N > 0 && items[k].lay.kind != G_LOCALARS) order[no++] = &items[k];
+  }
+  auto cost = [](const TrGenItem<T> *x) { return x->lay.N * size_t(x->lay.a.L + x->lay.b.L + 4); };
+  std::sort(order, order + no, [&](const TrGenItem<T> *x, const TrGenItem<T> *y) {
+    return cost(x) != cost(y) ? cost(x) > cost(y) : x < y;
+  });
+  TrGenArgs<T> ka;
+  ka.keys = tr_keys(L, seed);
+  for (size_t first = 0; first < no; first += kGenGates) {
+    ka.ng = int(std::min<size_t>(kGenGates, no - first));
+    ka.tiles = 0;
+    for (int k = 0; k < ka.ng; k++) {
+      const TrGenItem<T> &it = *order[first + size_t(k)];
+      ka.g[k].a = tr_gen_args(it.lay, it.gate, it.in, it.out, k0, k1);
+      ka.g[k].tile0 = ka.tiles;
+      ka.g[k].has_rout = 1;
+      ka.tiles += (it.lay.N + 63) / 64;
+    }
+    const hipError_t e = tr_gen_launch(L, ka);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 // A gate evaluation of fewer elements than this is latency-bound (a few
@@ -1201,6 +1290,9 @@ hipError_t launch_tr_expand(const Launch &L, const TrLayout &lay, const uint8_t 
 #define INST(T)                                                                                                       \
   template hipError_t launch_tr_keygen<T>(const Launch &, const TrLayout &, uint64_t, uint32_t, const T *, T *,       \
                                           uint8_t *, uint8_t *);                                                      \
+  template hipError_t launch_tr_masks<T>(const Launch &, uint64_t, const TrGenItem<T> *, size_t);                     \
+  template hipError_t launch_tr_keygen_batch<T>(const Launch &, uint64_t, const TrGenItem<T> *, size_t, uint8_t *,    \
+                                                uint8_t *);                                                           \
   template hipError_t launch_tr_expand<T>(const Launch &, const TrLayout &, const uint8_t *, uint32_t, int,           \
                                           uint8_t *);                                                                 \
   template hipError_t launch_tr_eval<T>(const Launch &, const TrLayout &, const uint8_t *, const uint8_t *,           \

@@ -114,6 +114,23 @@ struct TrPlan {
 template <typename T>
 hipError_t launch_tr_keygen(const Launch &L, const TrLayout &lay, uint64_t seed, uint32_t gate, const T *in_mask,
                             T *out_mask, uint8_t *k0, uint8_t *k1);
+// Several gates of one key set at once: the output masks of the gates are PRF
+// blocks, which no input mask enters, so a dealer draws them all first
+// (launch_tr_masks), forms the input masks from them, and then writes every
+// gate's keys (launch_tr_keygen_batch; lay holds offsets into k0 / k1).  Not for
+// G_DRELU, whose output mask depends on its input's.
+template <typename T>
+struct TrGenItem {
+  TrLayout lay;
+  uint32_t gate = 0;
+  const T *in = nullptr;
+  T *out = nullptr;
+};
+template <typename T>
+hipError_t launch_tr_masks(const Launch &L, uint64_t seed, const TrGenItem<T> *items, size_t n);
+template <typename T>
+hipError_t launch_tr_keygen_batch(const Launch &L, uint64_t seed, const TrGenItem<T> *items, size_t n, uint8_t *k0,
+                                  uint8_t *k1);
 // Regenerates into key (laid out by lay) the planes of party p's key of a
 // truncation-family gate that keygen drew from the party's own PRF key
 // (party_key): its DCF roots and output-mask bits, and for party 0 its shares
@@ -283,6 +300,9 @@ hipError_t launch_pool_diff(const Launch &L, int B, int R, int C, const T *V, T 
 // Vn[(b*Rn+j)*C+c] = V[(b*R+2j)*C+c] + y0[..] (+ y1[..]); carry the odd row
 template <typename T>
 hipError_t launch_pool_combine(const Launch &L, int B, int R, int C, const T *V, const T *y0, const T *y1, T *Vn);
+// The dealer's step of a level: D as launch_pool_diff, Vn as launch_pool_combine
+template <typename T>
+hipError_t launch_pool_masks(const Launch &L, int B, int R, int C, const T *V, const T *y, T *D, T *Vn);
 // concat rows: out[b*(w1+w2)+j] = j<w1 ? a[b*w1+j] : (bzero ? 0 : b[b*w2+j-w1])
 template <typename T>
 hipError_t launch_concat(const Launch &L, int B, int w1, int w2, const T *a, const T *b, T *out);

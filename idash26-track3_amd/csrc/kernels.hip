@@ -1007,6 +1007,32 @@ hipError_t launch_pool_combine(const Launch &L, int B, int R, int C, const T *V,
 }
 
 template <typename T>
+__global__ void k_pool_masks(int B, int R, int C, const T *V, const T *y, T *D, T *Vn) {
+  const int pr = R / 2, Rn = pr + (R & 1);
+  const size_t n = size_t(B) * Rn * C;
+  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) {
+    const size_t c = i % C, bj = i / C;
+    const size_t b = bj / Rn, j = bj % Rn;
+    const size_t o = (b * R + 2 * j) * C + c;
+    const T v = V[o];
+    if (int(j) < pr) {
+      const size_t k = (b * pr + j) * C + c;
+      D[k] = V[o + C] - v;
+      Vn[i] = v + y[k];
+    } else {
+      Vn[i] = v;
+    }
+  }
+}
+template <typename T>
+hipError_t launch_pool_masks(const Launch &L, int B, int R, int C, const T *V, const T *y, T *D, T *Vn) {
+  const int block = 256;
+  const int grid = grid_for(k_pool_masks<T>, block, size_t(B) * (R / 2 + (R & 1)) * C, L.num_cu);
+  hipLaunchKernelGGL((k_pool_masks<T>), dim3(grid), dim3(block), 0, L.stream, B, R, C, V, y, D, Vn);
+  return hipGetLastError();
+}
+
+template <typename T>
 __global__ void k_concat(int B, int w1, int w2, const T *a, const T *b, T *out) {
   const int w = w1 + w2;
   const size_t n = size_t(B) * w;
@@ -1098,6 +1124,7 @@ hipError_t launch_rowsum(const Launch &L, size_t rows, int len, const T *a, T *o
   template hipError_t launch_pool_prep<T>(const Launch &, size_t, int, const T *, const T *, T, T, T *);              \
   template hipError_t launch_pool_diff<T>(const Launch &, int, int, int, const T *, T *);                             \
   template hipError_t launch_pool_combine<T>(const Launch &, int, int, int, const T *, const T *, const T *, T *);    \
+  template hipError_t launch_pool_masks<T>(const Launch &, int, int, int, const T *, const T *, T *, T *);    \
   template hipError_t launch_concat<T>(const Launch &, int, int, int, const T *, const T *, T *);                     \
   template hipError_t launch_output<T>(const Launch &, int, int, int, const T *, const T *, int64_t, int64_t *);      \
   template hipError_t launch_rowsum<T>(const Launch &, size_t, int, const T *, T *);

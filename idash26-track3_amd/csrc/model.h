@@ -95,7 +95,9 @@ class ModelBase {
  public:
   virtual ~ModelBase() = default;
   virtual size_t key_bytes(int B) const = 0;
-  virtual hipError_t keygen(int B, uint64_t seed) = 0;
+  // a dealer run, enqueued on the lane's stream, and its completion
+  virtual hipError_t keygen_begin(int B, uint64_t seed) = 0;
+  virtual hipError_t keygen_end(int B, uint64_t seed) = 0;
   virtual hipError_t import_keys(int B, const void *k0, const void *k1, size_t bytes) = 0;
   virtual hipError_t export_keys(int party, void *dst, size_t bytes) = 0;
   virtual hipError_t release_arena() = 0;

@@ -518,6 +518,51 @@ struct Runner {
 // ---------------------------------------------------------------------------
 // dealer: keys of gates at a cursor, written into resident arenas
 // ---------------------------------------------------------------------------
+// Device memory of a dealer run, kept between runs: take() hands out ranges in
+// order, and a run of the same sizes gets the ranges of the one before.
+template <typename T>
+struct MaskPool {
+  struct Chunk {
+    DevBuf<T> buf;
+    size_t n = 0;
+  };
+  std::vector<std::unique_ptr<Chunk>> chunks;
+  size_t cur = 0, off = 0;
+  void reset() { cur = off = 0; }
+  void release() {
+    chunks.clear();
+    reset();
+  }
+  hipError_t take(size_t n, T **p) {
+    constexpr size_t kUnit = 256 / sizeof(T), kChunk = (size_t(16) << 20) / sizeof(T);
+    n = (n + kUnit - 1) / kUnit * kUnit;
+    while (cur < chunks.size() && off + n > chunks[cur]->n) {
+      cur++;
+      off = 0;
+    }
+    if (cur == chunks.size()) {
+      auto c = std::make_unique<Chunk>();
+      const size_t want = std::max(n, kChunk);
+      TRY(c->buf.alloc(want));
+      c->n = want;
+      chunks.push_back(std::move(c));
+    }
+    *p = chunks[cur]->buf.p + off;
+    off += n;
+    return hipSuccess;
+  }
+};
+
+// With a batch set, the truncation-family gates' keys are not written gate by
+// gate: their output masks were drawn before the run (items, in gate order), tr()
+// notes each gate's input mask, and the caller writes all keys at the end
+// (launch_tr_keygen_batch).  A key set's small gates then share launches instead
+// of each costing its chain of PRF blocks and hashes, and nothing waits for keys.
+template <typename T>
+struct GenBatch {
+  std::vector<TrGenItem<T>> items;
+  size_t next = 0;
+};
 template <typename T>
 struct Dealer {
   const Launch &L;
@@ -525,6 +570,7 @@ struct Dealer {
   uint64_t seed;
   uint8_t *K0, *K1;
   Cursor c;
+  GenBatch<T> *batch = nullptr;
 
   hipError_t reveal(size_t n, T *mask) {
     RevealLayout lay = reveal_layout(bw, n, c.off);
@@ -533,9 +579,19 @@ struct Dealer {
     c.gate++;
     return hipSuccess;
   }
-  hipError_t tr(int kind, size_t n, const T *in, T *out) {
+  // own: the output mask's place without a batch; *out: where it is
+  hipError_t tr(int kind, size_t n, const T *in, T *own, const T **out) {
     TrLayout lay = tr_layout(kind, bw, s, n, c.off);
-    TRY(launch_tr_keygen<T>(L, lay, seed, c.gate, in, out, K0, K1));
+    if (batch) {
+      if (batch->next >= batch->items.size()) return hipErrorUnknown;
+      TrGenItem<T> &it = batch->items[batch->next++];
+      if (it.gate != c.gate || it.lay.kind != kind || it.lay.N != n || it.lay.end != lay.end) return hipErrorUnknown;
+      it.in = in;
+      *out = it.out;
+    } else {
+      TRY(launch_tr_keygen<T>(L, lay, seed, c.gate, in, own, K0, K1));
+      *out = own;
+    }
     c.off = lay.end;
     c.gate++;
     return hipSuccess;
@@ -649,8 +705,9 @@ struct AdjNorm {
     TRY(d.reveal(BN, t0.p));                                // degree mask
     TRY(d.lut8(BN, t0.p, t1.p));                            // mask of T[d]
     TRY(d.mul(BN, BN, BP, MulMap::of(MulMap::OUTER_TRI, N), t1.p, t1.p, p0.p));  // mask of the outer product
-    TRY(d.tr(G_TRSLACK, BP, p0.p, p1.p));                    // mask of W
-    TRY(d.mul(BNN, BP, BNN, MulMap::of(MulMap::SYM_HADAMARD, N), rA, p1.p, rN));  // mask of A_norm
+    const T *w = nullptr;
+    TRY(d.tr(G_TRSLACK, BP, p0.p, p1.p, &w));  // mask of W
+    TRY(d.mul(BNN, BP, BNN, MulMap::of(MulMap::SYM_HADAMARD, N), rA, w, rN));  // mask of A_norm
     return hipSuccess;
   }
 
@@ -733,7 +790,7 @@ class Model final : public ModelBase, KeySource {
   // in gpuReluExtend (:225-234): 6 + 13 AES per element and party at bw=32
   // instead of 31 for one fused gate over the full width.  With local
   // truncation: the local shift (no key) followed, for relu, by a RELU gate.
-  // Eval may overwrite x; keygen may overwrite the mask rin.
+  // Eval may overwrite x.
   hipError_t trunc_eval(Runner<T> &r, bool relu, size_t n, T *x, const T *bias, int ncol, T *y) {
     if (!local_trunc()) {
       if (n <= r.pair_max) return r.tr2(G_TRMOD, relu ? G_EXTRELU : G_EXT, n, x, bias, ncol, y);
@@ -743,13 +800,17 @@ class Model final : public ModelBase, KeySource {
     TRY(launch_local_ars<T>(L_, n, s_, x, bias, ncol, relu ? x : y));
     return relu ? r.tr(G_RELU, n, x, nullptr, 1, y) : hipSuccess;
   }
-  hipError_t trunc_keygen(Dealer<T> &d, bool relu, size_t n, T *rin, T *rout) {
+  hipError_t trunc_keygen(Dealer<T> &d, bool relu, size_t n, const T *rin, const T **rout) {
     if (!local_trunc()) {
-      TRY(d.tr(G_TRMOD, n, rin, rin));
-      return d.tr(relu ? G_EXTRELU : G_EXT, n, rin, rout);
+      const T *y = nullptr;
+      TRY(d.tr(G_TRMOD, n, rin, nullptr, &y));
+      return d.tr(relu ? G_EXTRELU : G_EXT, n, y, nullptr, rout);
     }
-    TRY(launch_local_ars<T>(L_, n, s_, rin, nullptr, 1, relu ? rin : rout));
-    return relu ? d.tr(G_RELU, n, rin, rout) : hipSuccess;
+    T *y = nullptr;
+    TRY(gen_.take(n, &y));
+    TRY(launch_local_ars<T>(L_, n, s_, rin, nullptr, 1, y));
+    *rout = y;
+    return relu ? d.tr(G_RELU, n, y, nullptr, rout) : hipSuccess;
   }
 
   // ---------------- weights ----------------
@@ -898,6 +959,7 @@ class Model final : public ModelBase, KeySource {
   hipError_t release_arena() override {
     TRY(hipStreamSynchronize(L_.stream));
     free_arena();
+    gen_.release();
     if (!streaming_) keyed_B_ = -1;
     return hipSuccess;
   }
@@ -955,94 +1017,115 @@ class Model final : public ModelBase, KeySource {
     return hipSuccess;
   }
 
-  hipError_t keygen(int B, uint64_t seed) override {
+  // Enqueues a dealer run on the lane's stream; keygen_end waits for it.
+  hipError_t keygen_begin(int B, uint64_t seed) override {
     if (party_ >= 0) return hipErrorNotSupported;  // the dealer holds both parties' keys
     TRY(leave_stream());
     keyed_B_ = -1;  // until the new keys are complete
+    have_pk_ = false;
     TRY(hipStreamSynchronize(L_.stream));  // a running forward may still read the arena
     drop_graph();
     TRY(ensure_arena(B));
     TRY(ensure_work(B));
     const int N = d_.n_nodes;
     const size_t BN = size_t(B) * N, BNN = BN * N;
-    const size_t E = emax(B);
-    DevBuf<T> rX, t1, t2, rA, rN, rm, gt;
-    TRY(rX.alloc(E));
-    TRY(t1.alloc(E));
-    TRY(t2.alloc(E));
-    TRY(rA.alloc(BNN));
-    TRY(rN.alloc(BNN));
-    TRY(rm.alloc(BN));
-    TRY(gt.alloc(E));
-    Dealer<T> d{L_, bw_, s_, seed, arena_[0], arena_[1], Cursor{}};
-    auto pub_gemm = [&](const T *x, int l, size_t rows, T *y) -> hipError_t {
+    gen_.reset();
+    auto take = [&](size_t n, T **p) { return gen_.take(n, p); };
+    // every gate's output mask first: PRF blocks that depend on nothing
+    GenBatch<T> batch;
+    for (const GateKey &g : plan(B)) {
+      if (!g.tr_kind) continue;
+      TrGenItem<T> it;
+      it.lay = tr_layout(g.tr_kind, bw_, s_, g.n, g.begin);
+      it.gate = g.gate;
+      TRY(take(g.n, &it.out));
+      batch.items.push_back(it);
+    }
+    TRY(launch_tr_masks<T>(L_, seed, batch.items.data(), batch.items.size()));
+    Dealer<T> d{L_, bw_, s_, seed, arena_[0], arena_[1], Cursor{}, &batch};
+    auto pub_gemm = [&](const T *x, int l, size_t rows, T **y) -> hipError_t {
       int in, out;
       layer_io(l, &in, &out);
+      TRY(take(rows * size_t(out), y));
       GemmArgs<T> g;
       g.M = int(rows);
       g.K = in;
       g.N = out;
       g.A1 = x;
       g.B1 = wt_[l].p;
-      g.C = y;
+      g.C = *y;
       return launch_gemm<T>(L_, g);
     };
 
-    TRY(d.reveal(BN * d_.feat, rX.p));
-    TRY(d.reveal(BN, rm.p));
-    TRY(adj_.keygen(d, rA.p, rN.p));
-    // GCN stack; rX holds the running activation mask
+    T *rX, *rm, *rA, *rN, *tmp, *z;
+    TRY(take(BN * d_.feat, &rX));
+    TRY(take(BN, &rm));
+    TRY(take(BNN, &rA));
+    TRY(take(BNN, &rN));
+    TRY(take(BN * size_t(std::max(d_.gcn[0], std::max(d_.gcn[1], d_.gcn[2]))), &tmp));
+    TRY(d.reveal(BN * d_.feat, rX));
+    TRY(d.reveal(BN, rm));
+    TRY(adj_.keygen(d, rA, rN));
+    // GCN stack; x is the running activation mask
+    const T *x = rX, *y = nullptr;
     for (int l = 0; l < 3; l++) {
       const int fo = d_.gcn[l];
       const size_t En = BN * fo;
-      TRY(pub_gemm(rX.p, l, BN, t1.p));
+      TRY(pub_gemm(x, l, BN, &z));
       if (xw_slack())
-        TRY(d.tr(G_TRSLACK, En, t1.p, t2.p));
+        TRY(d.tr(G_TRSLACK, En, z, nullptr, &y));
       else
-        TRY(trunc_keygen(d, false, En, t1.p, t2.p));
-      TRY(d.sxs(B, N, N, fo, rN.p, t2.p, t1.p, gt.p));
+        TRY(trunc_keygen(d, false, En, z, &y));
+      TRY(take(En, &z));
+      TRY(d.sxs(B, N, N, fo, rN, y, z, tmp));
       if (agg_split()) {
-        TRY(d.tr(G_TRSLACK, En, t1.p, t2.p));
-        TRY(d.tr(G_RELUSLACK, En, t2.p, rX.p));
+        TRY(d.tr(G_TRSLACK, En, z, nullptr, &y));
+        TRY(d.tr(G_RELUSLACK, En, y, nullptr, &x));
       } else {
-        TRY(trunc_keygen(d, true, En, t1.p, rX.p));
+        TRY(trunc_keygen(d, true, En, z, &x));
       }
     }
     // pool
     const int C = d_.gcn[2];
     const T Sm = T(1) << (pool_sentinel_bit() - d_.mask_scale);
-    TRY(launch_pool_prep<T>(L_, BN, C, rX.p, rm.p, Sm, T(0), t2.p));  // rV in t2
-    T *cur = t2.p, *nxt = rX.p;
+    T *cur, *dm, *nxt;
+    TRY(take(BN * C, &cur));
+    TRY(launch_pool_prep<T>(L_, BN, C, x, rm, Sm, T(0), cur));
     int pairs[32];
     const int Lv = pool_levels(N, pairs);
     int R = N;
     for (int l = 0; l < Lv; l++) {
       const int pr = pairs[l];
       const size_t En = size_t(B) * pr * C;
-      TRY(launch_pool_diff<T>(L_, B, R, C, cur, t1.p));
-      TRY(d.tr(pool_kind(), En, t1.p, gt.p));
-      TRY(launch_pool_combine<T>(L_, B, R, C, cur, gt.p, nullptr, nxt));
-      std::swap(cur, nxt);
+      TRY(take(En, &dm));
+      TRY(take(size_t(B) * (pr + (R & 1)) * C, &nxt));
+      TRY(d.tr(pool_kind(), En, dm, nullptr, &y));
+      TRY(launch_pool_masks<T>(L_, B, R, C, cur, y, dm, nxt));
+      cur = nxt;
       R = pr + (R & 1);
     }
     // drug FCs
-    TRY(pub_gemm(cur, 3, B, t1.p));
-    TRY(trunc_keygen(d, true, size_t(B) * d_.dfc[0], t1.p, gt.p));
-    TRY(pub_gemm(gt.p, 4, B, t1.p));
-    TRY(trunc_keygen(d, false, size_t(B) * d_.dfc[1], t1.p, gt.p));
-    TRY(launch_concat<T>(L_, B, d_.dfc[1], d_.prot, gt.p, nullptr, nxt));
-    T *h = nxt, *h2 = cur;
+    TRY(pub_gemm(cur, 3, B, &z));
+    TRY(trunc_keygen(d, true, size_t(B) * d_.dfc[0], z, &x));
+    TRY(pub_gemm(x, 4, B, &z));
+    TRY(trunc_keygen(d, false, size_t(B) * d_.dfc[1], z, &x));
+    T *h;
+    TRY(take(size_t(B) * (d_.dfc[1] + d_.prot), &h));
+    TRY(launch_concat<T>(L_, B, d_.dfc[1], d_.prot, x, nullptr, h));
+    x = h;
     for (int k = 0; k < d_.nfus; k++) {
-      TRY(pub_gemm(h, 5 + k, B, t1.p));
-      if (k < d_.nfus - 1) {
-        TRY(trunc_keygen(d, true, size_t(B) * d_.fus[k], t1.p, h2));
-        std::swap(h, h2);
-      } else {
-        TRY(d.output(size_t(B) * d_.fus[k], t1.p));
-      }
+      TRY(pub_gemm(x, 5 + k, B, &z));
+      if (k < d_.nfus - 1)
+        TRY(trunc_keygen(d, true, size_t(B) * d_.fus[k], z, &x));
+      else
+        TRY(d.output(size_t(B) * d_.fus[k], z));
     }
     // plan and dealer disagree (offsets, or gate ids of the seeded-plane expansion)
-    if (d.c.off != key_bytes(B) || d.c.gate != uint32_t(plan(B).size()) + 1) return hipErrorUnknown;
+    if (d.c.off != key_bytes(B) || d.c.gate != uint32_t(plan(B).size()) + 1 || batch.next != batch.items.size())
+      return hipErrorUnknown;
+    return launch_tr_keygen_batch<T>(L_, seed, batch.items.data(), batch.items.size(), arena_[0], arena_[1]);
+  }
+  hipError_t keygen_end(int B, uint64_t seed) override {
     TRY(hipStreamSynchronize(L_.stream));
     for (int p = 0; p < 2; p++) party_key_bytes(L_, seed, p, pk_[p]);
     have_pk_ = true;
@@ -1791,6 +1874,7 @@ class Model final : public ModelBase, KeySource {
   DevBuf<int64_t> out_;
   Workspace<T> ws_;
   AdjNorm<T> adj_;
+  MaskPool<T> gen_;  // a dealer run's masks
   // gate plan and streaming state
   std::vector<GateKey> gates_;
   std::vector<std::pair<size_t, size_t>> chunks_;
@@ -1957,7 +2041,13 @@ size_t LaneSet::unique_key_bytes(int B, int party) const {
 
 hipError_t LaneSet::keygen(int B, uint64_t seed) {
   keyed_B_ = -1;
-  TRY(each(B, [&](int i, int Bi, int) { return lane_[i]->keygen(Bi, lane_seed(seed, i)); }));
+  // the lanes' runs side by side, then waited for; a failed run leaves none behind
+  hipError_t e = each(B, [&](int i, int Bi, int) { return lane_[i]->keygen_begin(Bi, lane_seed(seed, i)); });
+  if (e != hipSuccess) {
+    for (size_t i = 0; i < st_.size(); i++) (void)hipStreamSynchronize(st_[i]);
+    return e;
+  }
+  TRY(each(B, [&](int i, int Bi, int) { return lane_[i]->keygen_end(Bi, lane_seed(seed, i)); }));
   keyed_B_ = B;
   return hipSuccess;
 }
