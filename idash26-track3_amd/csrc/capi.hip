@@ -11,6 +11,7 @@
 #include "../../include/mpcx.h"
 #include "gemm.h"
 #include "kernels.h"
+#include "launch_util.h"
 #include "model.h"
 #include "mpcx_core.h"
 #include "peer.h"
@@ -731,6 +732,19 @@ template <typename T>
 static mpcx_status mul_eval_t(mpcx_ctx *c, size_t nx, size_t ny, size_t nz, const uint32_t *ia, const uint32_t *ib,
                               const void *k0, const void *k1, const void *x, const void *y, void *z) {
   MulLayout lay = mul_layout(c->bw, nx, ny, nz, 0);
+  const size_t nb = nz * sizeof(T);
+  if (bytes_apart(z, nb, x, nx * sizeof(T)) && bytes_apart(z, nb, y, ny * sizeof(T)) && bytes_apart(z, nb, ia, 4 * nz) &&
+      bytes_apart(z, nb, ib, 4 * nz) && bytes_apart(z, nb, k0, lay.end) && bytes_apart(z, nb, k1, lay.end)) {
+    HIPC(c,
+         launch_mul_eval_sum<T>(c->L, lay, static_cast<const uint8_t *>(k0), static_cast<const uint8_t *>(k1),
+                                MulMap::explicit_maps(ia, ib), static_cast<const T *>(x), static_cast<const T *>(y),
+                                static_cast<T *>(z)),
+         "mul_eval");
+    c->counters.msg(nz, c->bw);
+    HIPC(c, hipStreamSynchronize(c->L.stream), "sync");
+    return MPCX_OK;
+  }
+  // the output overlaps an operand, which other threads gather: the messages first
   void *sp = nullptr;
   HIPC(c, ctx_work(c, 2 * nz * sizeof(T), &sp), "hipMalloc");
   T *m0 = static_cast<T *>(sp), *m1 = m0 + nz;
@@ -787,6 +801,19 @@ template <typename T>
 static mpcx_status lut_eval_t(mpcx_ctx *c, size_t n, const void *k0, const void *k1, const void *table, const void *x,
                               void *y) {
   Lut8Layout lay = lut8_layout(c->bw, n, 0);
+  const size_t nb = n * sizeof(T);
+  if ((x == y || bytes_apart(y, nb, x, nb)) && bytes_apart(y, nb, table, 256 * sizeof(T)) &&
+      bytes_apart(y, nb, k0, lay.end) && bytes_apart(y, nb, k1, lay.end)) {
+    HIPC(c,
+         launch_lut8_sum<T>(c->L, lay, static_cast<const uint8_t *>(k0), static_cast<const uint8_t *>(k1),
+                            static_cast<const T *>(table), static_cast<const T *>(x), static_cast<T *>(y)),
+         "lut8_eval");
+    c->counters.msg(n, c->bw);
+    c->counters.msg(n, c->bw);
+    HIPC(c, hipStreamSynchronize(c->L.stream), "sync");
+    return MPCX_OK;
+  }
+  // the output overlaps an input: the messages first
   void *sp = nullptr;
   HIPC(c, ctx_work(c, 3 * n * sizeof(T), &sp), "hipMalloc");
   T *m0 = static_cast<T *>(sp), *m1 = m0 + n, *vh = m1 + n;
@@ -987,6 +1014,18 @@ template <typename T>
 static mpcx_status reveal_eval_t(mpcx_ctx *c, size_t n, const void *k0, const void *k1, const void *v0,
                                  const void *v1, void *out) {
   RevealLayout lay = reveal_layout(c->bw, n, 0);
+  const size_t nb = n * sizeof(T);
+  if ((out == v0 || bytes_apart(out, nb, v0, nb)) && (out == v1 || bytes_apart(out, nb, v1, nb)) &&
+      bytes_apart(out, nb, k0, lay.end) && bytes_apart(out, nb, k1, lay.end)) {
+    HIPC(c,
+         launch_reveal_sum<T>(c->L, lay, static_cast<const uint8_t *>(k0), static_cast<const uint8_t *>(k1),
+                              static_cast<const T *>(v0), static_cast<const T *>(v1), 0, static_cast<T *>(out)),
+         "reveal_eval");
+    c->counters.msg(n, c->bw);
+    HIPC(c, hipStreamSynchronize(c->L.stream), "sync");
+    return MPCX_OK;
+  }
+  // the output overlaps a share elsewhere: the messages first
   void *sp = nullptr;
   HIPC(c, ctx_work(c, 2 * n * sizeof(T), &sp), "hipMalloc");
   T *m0 = static_cast<T *>(sp), *m1 = m0 + n;

@@ -79,6 +79,7 @@ __device__ __forceinline__ void pool_carry(const TrPool<T> &q) {
   }
 }
 
+__device__ __forceinline__ bool tr_is_ext(int kind) { return kind == G_EXT || kind == G_EXTRELU; }
 __device__ __forceinline__ bool relu_like(int kind) {
   return kind == G_RELU || kind == G_RELUSLACK || kind == G_RELUPOOL;
 }
@@ -133,32 +134,31 @@ __device__ __forceinline__ void tr_dcf_bits(const Aes &aes, const TrArgs<T> &a, 
 // reconstructed masked bits of planes a and b.  The two parties' messages add
 // up to the masked output.
 template <typename T>
+__device__ __forceinline__ uint32_t tr_case(const TrArgs<T> &a, T xp, uint32_t hb, uint32_t bh, uint32_t dh) {
+  if (a.kind == G_TRMOD) return dh;
+  if (tr_is_ext(a.kind)) return hb * 2 + bh;
+  if (a.kind == G_TR || a.kind == G_TRRELU) return hb * 4 + bh * 2 + dh;
+  if (relu_like(a.kind)) return hb ^ bh;
+  if (a.kind == G_DRELU) return 0;  // no table
+  return (uint32_t(xp >> (a.n - 2)) & 3u) * 2 + dh;  // G_TRSLACK
+}
+// The message from the case's G word and (ReLU kinds) the kappa share; z = hb ^ bh.
+template <typename T>
+__device__ __forceinline__ T tr_message(const TrArgs<T> &a, int p, T xh, T xp, uint32_t z, T g, T k) {
+  const T one0 = p == 0 ? T(1) : T(0);
+  if (a.kind == G_DRELU) return one0 * T(z);  // the public masked bit; party 0 carries it
+  const T A = (xp >> a.sh) - (T(1) << (a.m - 1 - a.sh));
+  if (!a.relu) return one0 * A + g;  // TRMOD: exact modulo 2^(n-s), no wrap term
+  const T cp = z ? T(one0 - k) : k;
+  return cp * (relu_like(a.kind) ? xh : A) + g;
+}
+template <typename T>
 __device__ __forceinline__ T tr_out_share(const TrArgs<T> &a, int p, const uint8_t *K, size_t i, T xh, T xp,
                                           uint32_t hb, uint32_t bh, uint32_t dh) {
-  const T *G = reinterpret_cast<const T *>(K + a.off_g);
-  const T *kap = reinterpret_cast<const T *>(K + a.off_kappa);
-  const T one0 = p == 0 ? T(1) : T(0);
-  const T A = (xp >> a.sh) - (T(1) << (a.m - 1 - a.sh));
-  if (a.kind == G_TRMOD) return one0 * A + G[size_t(dh) * a.N + i];  // exact modulo 2^(n-s): no wrap term
-  if (a.kind == G_EXT) return one0 * A + G[size_t(hb * 2 + bh) * a.N + i];
-  if (a.kind == G_EXTRELU || a.kind == G_TRRELU) {
-    const uint32_t z = hb ^ bh;
-    const T k = kap[i];
-    const T cp = z ? T(one0 - k) : k;
-    const size_t c = a.kind == G_EXTRELU ? hb * 2 + bh : hb * 4 + bh * 2 + dh;
-    return cp * A + G[c * a.N + i];
-  }
-  if (a.kind == G_TR) return one0 * A + G[size_t(hb * 4 + bh * 2 + dh) * a.N + i];
-  if (a.kind == G_DRELU) return one0 * T(hb ^ bh);  // the public masked bit; party 0 carries it
-  if (relu_like(a.kind)) {
-    const uint32_t z = hb ^ bh;
-    const T k = kap[i];
-    const T cp = z ? T(one0 - k) : k;
-    return cp * xh + G[size_t(z) * a.N + i];
-  }
-  // G_TRSLACK
-  const uint32_t Hh = uint32_t(xp >> (a.n - 2)) & 3u;
-  return one0 * A + G[size_t(Hh * 2 + dh) * a.N + i];
+  T g = 0, k = 0;
+  if (a.ncase) g = reinterpret_cast<const T *>(K + a.off_g)[size_t(tr_case(a, xp, hb, bh, dh)) * a.N + i];
+  if (a.relu) k = reinterpret_cast<const T *>(K + a.off_kappa)[i];
+  return tr_message(a, p, xh, xp, hb ^ bh, g, k);
 }
 
 // The revealed output from the two parties' messages: their sum, reduced to
@@ -327,27 +327,44 @@ __device__ __forceinline__ void tr_eval_both(const TrArgs<T> &a, const TrArgs<T>
 }
 
 // ---- quad-lane form (latency-bound launches, AesPerm2 table) ----
-// The DCF walks of tr_dcf_bits with four lanes per element and party (lane j of
-// the quad reads word j of the roots, correction words and leaves).
+// What a gate reads from the keys before it can start, and at its end: the
+// lane's words of the roots, leaves and first correction words of its planes,
+// the mask bits, the lane's entry of the G table (lane j holds case j and, for
+// eight cases, 4 + j) and the kappa share.  A launch of few waves waits out every
+// load, so all go out at once, and those of a second gate (or a tree's next
+// level) while the first one runs.
 template <typename T>
-__device__ __forceinline__ void tr_dcf_bits_quad(const AesQuad &aes, const AesQuad::Keys &kH,
-                                                 const AesQuad::Keys &kL, const TrArgs<T> &a, const uint8_t *K,
-                                                 const uint8_t *KC, size_t i, T xp, uint32_t *ra, uint32_t *rb) {
-  const T lowmask = (T(1) << a.sb) - T(1);
-  const T smask = (T(1) << a.s) - T(1);
-  const size_t w = 4 * i + aes.j, sw = 4 * a.N;
+struct QuadKeys {
+  uint32_t sa = 0, la = 0, ca = 0, za = 0, sb = 0, lb = 0, cb = 0, zb = 0;
+  T g0 = 0, g1 = 0, kap = 0;
+};
+template <typename T>
+__device__ __forceinline__ QuadKeys<T> quad_keys(const TrArgs<T> &a, uint32_t j, const uint8_t *K, const uint8_t *KC,
+                                                 size_t i) {
+  QuadKeys<T> q;
+  const size_t w = 4 * i + j;
+  auto word = [&](const uint8_t *P, size_t off) { return reinterpret_cast<const uint32_t *>(P + off)[w]; };
   if (a.use_a) {
-    *ra = dcf_eval_walk_quad(aes, kH, kL, reinterpret_cast<const uint32_t *>(K + a.a.off_root)[w], a.a.m, a.a.L,
-                             reinterpret_cast<const uint32_t *>(KC + a.a.off_cw) + w, sw,
-                             reinterpret_cast<const uint32_t *>(KC + a.a.off_leaf)[w], uint64_t(xp & lowmask));
-    *ra ^= get_bit(reinterpret_cast<const uint64_t *>(K + a.a.off_z), i);
+    q.sa = word(K, a.a.off_root);
+    q.la = word(KC, a.a.off_leaf);
+    if (a.a.L > 0) q.ca = word(KC, a.a.off_cw);
+    q.za = get_bit(reinterpret_cast<const uint64_t *>(K + a.a.off_z), i);
   }
   if (a.use_b) {
-    *rb = dcf_eval_walk_quad(aes, kH, kL, reinterpret_cast<const uint32_t *>(K + a.b.off_root)[w], a.b.m, a.b.L,
-                             reinterpret_cast<const uint32_t *>(KC + a.b.off_cw) + w, sw,
-                             reinterpret_cast<const uint32_t *>(KC + a.b.off_leaf)[w], uint64_t(xp & smask));
-    *rb ^= get_bit(reinterpret_cast<const uint64_t *>(K + a.b.off_z), i);
+    q.sb = word(K, a.b.off_root);
+    q.lb = word(KC, a.b.off_leaf);
+    if (a.b.L > 0) q.cb = word(KC, a.b.off_cw);
+    q.zb = get_bit(reinterpret_cast<const uint64_t *>(K + a.b.off_z), i);
   }
+  const T *G = reinterpret_cast<const T *>(K + a.off_g);
+  if (int(j) < a.ncase) q.g0 = G[size_t(j) * a.N + i];
+  if (a.ncase > 4) q.g1 = G[size_t(j + 4) * a.N + i];
+  if (a.relu) q.kap = reinterpret_cast<const T *>(K + a.off_kappa)[i];
+  return q;
+}
+__device__ __forceinline__ uint32_t quad_xor_all(uint32_t v) { return AesQuad::quad_xor(v); }
+__device__ __forceinline__ uint64_t quad_xor_all(uint64_t v) {
+  return uint64_t(AesQuad::quad_xor(uint32_t(v))) | (uint64_t(AesQuad::quad_xor(uint32_t(v >> 32))) << 32);
 }
 
 // tr_tile with a quad of lanes per element and party: the quad's lanes carry the
@@ -355,13 +372,23 @@ __device__ __forceinline__ void tr_dcf_bits_quad(const AesQuad &aes, const AesQu
 // every lane of the quad forms the message, the first one writes it.
 template <typename T>
 __device__ __forceinline__ T tr_tile_quad(const AesQuad &aes, const AesQuad::Keys &kH, const AesQuad::Keys &kL,
-                                          const TrArgs<T> &a, TrXchg<T> &x, int p, int e, int wv, const uint8_t *K,
-                                          const uint8_t *KC, size_t i, bool in, T xh) {
+                                          const TrArgs<T> &a, TrXchg<T> &x, int p, int e, int wv,
+                                          const QuadKeys<T> &k, const uint8_t *KC, size_t i, bool in, T xh) {
   uint32_t ra = 0, rb = 0;
   T xp = 0;
   if (in) {
     xp = tr_shifted_input(a, i, xh);
-    tr_dcf_bits_quad(aes, kH, kL, a, K, KC, i, xp, &ra, &rb);
+    const T lowmask = (T(1) << a.sb) - T(1);
+    const T smask = (T(1) << a.s) - T(1);
+    const size_t w = 4 * i + aes.j, sw = 4 * a.N;
+    if (a.use_a)
+      ra = dcf_eval_walk_quad(aes, kH, kL, k.sa, a.a.m, a.a.L, k.ca,
+                              reinterpret_cast<const uint32_t *>(KC + a.a.off_cw) + w, sw, k.la, T(xp & lowmask)) ^
+           k.za;
+    if (a.use_b)
+      rb = dcf_eval_walk_quad(aes, kH, kL, k.sb, a.b.m, a.b.L, k.cb,
+                              reinterpret_cast<const uint32_t *>(KC + a.b.off_cw) + w, sw, k.lb, T(xp & smask)) ^
+           k.zb;
   }
   const uint64_t wa = __ballot(ra), wb = __ballot(rb);
   if (lane_id() == 0) {
@@ -374,7 +401,10 @@ __device__ __forceinline__ T tr_tile_quad(const AesQuad &aes, const AesQuad::Key
     const uint32_t hb = uint32_t(xp >> a.sb) & 1u;
     const uint32_t bh = a.use_a ? uint32_t((x.xa[0][wv] ^ x.xa[1][wv]) >> q0) & 1u : 0u;
     const uint32_t dh = a.use_b ? uint32_t((x.xb[0][wv] ^ x.xb[1][wv]) >> q0) & 1u : 0u;
-    const T msg = tr_out_share(a, p, K, i, xh, xp, hb, bh, dh);
+    const uint32_t c = tr_case(a, xp, hb, bh, dh);
+    const T gj = c < 4 ? k.g0 : k.g1;
+    const T g = quad_xor_all((c & 3u) == aes.j ? gj : T(0));
+    const T msg = tr_message(a, p, xh, xp, hb ^ bh, g, k.kap);
     if ((lane_id() & 3u) == 0) x.xm[p][e] = msg;
   }
   __syncthreads();
@@ -405,7 +435,9 @@ __device__ __forceinline__ void tr_eval_tiles_quad(const TrArgs<T> &a, const TrA
     const bool in = i < a.N;
     T xin = 0, v0 = 0;
     uint32_t o = 0;
+    QuadKeys<T> qk, qk2;
     if (in) {
+      qk = quad_keys(a, aes.j, K, KC, i);
       if constexpr (POOL) {
         const uint32_t s0 = pool_src(q, uint32_t(i), &o);
         v0 = q.v[s0];
@@ -413,9 +445,10 @@ __device__ __forceinline__ void tr_eval_tiles_quad(const TrArgs<T> &a, const TrA
       } else {
         xin = a.xhat[i];
       }
+      if constexpr (TWO) qk2 = quad_keys(a2, aes.j, K, KC, i);
     }
-    T y = tr_tile_quad(aes, kH, kL, a, x, p, e, wv, K, KC, i, in, xin);
-    if constexpr (TWO) y = tr_tile_quad(aes, kH, kL, a2, x, p, e, wv, K, KC, i, in, y);
+    T y = tr_tile_quad(aes, kH, kL, a, x, p, e, wv, qk, KC, i, in, xin);
+    if constexpr (TWO) y = tr_tile_quad(aes, kH, kL, a2, x, p, e, wv, qk2, KC, i, in, y);
     if (p == 0 && in && (lt & 3) == 0) {
       if constexpr (POOL)
         q.vn[o] = v0 + y;
@@ -511,7 +544,8 @@ __global__ void k_tr_eval_pool_tail_q(TrTail<T> t) {
         v0 = vin[cc * R0 + 2 * j];
         xin = vin[cc * R0 + 2 * j + 1] - v0;
       }
-      const T y = tr_tile_quad(aes, kH, kL, a, x, p, e, wv, K, KC, i, in, xin);
+      const QuadKeys<T> qk = in ? quad_keys(a, aes.j, K, KC, i) : QuadKeys<T>{};
+      const T y = tr_tile_quad(aes, kH, kL, a, x, p, e, wv, qk, KC, i, in, xin);
       if (p == 0 && in && (lt & 3) == 0) vout[cc * R0 + j] = v0 + y;
     }
     if (R & 1)
@@ -628,20 +662,9 @@ struct TrGenArgs {
   size_t tiles = 0;
 };
 
-// A value in uniform, unwritten memory (kernel arguments), read into scalar
-// registers.  fresh() hides where a pointer comes from, so that what
-// is read through it is read there: round keys of three keys at once would not
-// fit the scalar registers and be spilled to vector lanes.
-using ConstWord = const __attribute__((address_space(4))) uint32_t;
-template <class S>
-__device__ __forceinline__ S load_uniform(ConstWord *p) {
-  uint32_t w[sizeof(S) / 4];
-#pragma unroll
-  for (size_t k = 0; k < sizeof(S) / 4; k++) w[k] = p[k];
-  S s;
-  __builtin_memcpy(&s, w, sizeof(S));
-  return s;
-}
+// Hides where a pointer to uniform memory comes from, so that what is read
+// through it is read there: round keys of three keys at once would not fit the
+// scalar registers and be spilled to vector lanes.
 __device__ __forceinline__ ConstWord *fresh(ConstWord *p) {
   asm volatile("" : "+s"(p));
   return p;

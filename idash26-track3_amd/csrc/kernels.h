@@ -267,6 +267,12 @@ template <typename T>
 hipError_t launch_lut8_phase2(const Launch &L, const Lut8Layout &lay, const uint8_t *k0, const uint8_t *k1,
                               const T *vhat, T *msg0, T *msg1);
 
+// Both parties in this process: the whole gate in one launch, the revealed
+// output in out (which may be xhat, but overlap neither it otherwise nor the table).
+template <typename T>
+hipError_t launch_lut8_sum(const Launch &L, const Lut8Layout &lay, const uint8_t *k0, const uint8_t *k1,
+                           const T *table, const T *xhat, T *out);
+
 // ---------------- SxS keys ----------------
 template <typename T>
 hipError_t launch_split(const Launch &L, uint64_t seed, uint32_t gate, uint32_t field, size_t n, const T *v,

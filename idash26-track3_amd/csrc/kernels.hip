@@ -654,16 +654,34 @@ hipError_t launch_mul_eval(const Launch &L, const MulLayout &lay, const uint8_t 
 // x^y^ - x^ ry0 - y^ rx0 + c0 and party 1's - x^ ry1 - y^ rx1 + c1, each from the
 // party's own key, and writes their sum, the revealed product (the operands are
 // read once, no message planes, no reconstruction launch).
+// kMulUnroll products a thread at once, so that their gathers are in flight
+// together (indices first, then the operands and masks at them).
+constexpr int kMulUnroll = 4;
 template <typename T>
 __global__ void k_mul_eval_sum(size_t nz, const T *Rx0, const T *Rx1, const T *Ry0, const T *Ry1, const T *C0,
                                const T *C1, MulMap map, const T *xhat, const T *yhat, T *out) {
-  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < nz; i += size_t(gridDim.x) * blockDim.x) {
-    uint32_t a, b;
-    mul_operands(map, i, &a, &b);
-    const T x = xhat[a], y = yhat[b];
-    const T z0 = C0[i] - x * Ry0[b] - y * Rx0[a] + x * y;
-    const T z1 = C1[i] - x * Ry1[b] - y * Rx1[a];
-    out[i] = z0 + z1;
+  const size_t tile = size_t(blockDim.x) * kMulUnroll;
+  for (size_t base = size_t(blockIdx.x) * tile + threadIdx.x; base < nz; base += size_t(gridDim.x) * tile) {
+    uint32_t a[kMulUnroll], b[kMulUnroll];
+    T z[kMulUnroll];
+#pragma unroll
+    for (int u = 0; u < kMulUnroll; u++) {
+      const size_t i = base + size_t(u) * blockDim.x, k = i < nz ? i : nz - 1;
+      mul_operands(map, k, &a[u], &b[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kMulUnroll; u++) {
+      const size_t i = base + size_t(u) * blockDim.x, k = i < nz ? i : nz - 1;
+      const T x = xhat[a[u]], y = yhat[b[u]];
+      const T z0 = C0[k] - x * Ry0[b[u]] - y * Rx0[a[u]] + x * y;
+      const T z1 = C1[k] - x * Ry1[b[u]] - y * Rx1[a[u]];
+      z[u] = z0 + z1;
+    }
+#pragma unroll
+    for (int u = 0; u < kMulUnroll; u++) {
+      const size_t i = base + size_t(u) * blockDim.x;
+      if (i < nz) out[i] = z[u];
+    }
   }
 }
 
@@ -745,14 +763,21 @@ hipError_t launch_mul_eval_sum(const Launch &L, const MulLayout &lay, const uint
   if (map.kind == MulMap::SYM_HADAMARD && 3 * TI * size_t(map.N) * sizeof(T) <= 65536) {
     const size_t N = map.N, NN = N * N, P = N * (N + 1) / 2;
     if (N == 0 || lay.nz % NN != 0 || lay.nx != lay.nz || lay.ny != (lay.nz / NN) * P) return hipErrorInvalidValue;
-    const size_t tiles = (N + TI - 1) / TI, blocks = (lay.nz / NN) * tiles;
-    if (blocks >= (size_t(1) << 31)) return hipErrorInvalidValue;
-    const size_t lds = 3 * TI * N * sizeof(T);
-    hipLaunchKernelGGL((k_mul_eval_sym_sum<T, TI>), dim3(unsigned(blocks)), dim3(block), lds, L.stream, uint32_t(N),
-                       Rx0, Rx1, Ry0, Ry1, C0, C1, xhat, yhat, out);
-    return hipGetLastError();
+    const size_t graphs = lay.nz / NN;
+    auto go = [&](auto ti) {
+      constexpr int R = decltype(ti)::value;
+      const size_t blocks = graphs * ((N + R - 1) / R);
+      if (blocks >= (size_t(1) << 31)) return hipErrorInvalidValue;
+      hipLaunchKernelGGL((k_mul_eval_sym_sum<T, R>), dim3(unsigned(blocks)), dim3(block), 3 * R * N * sizeof(T),
+                         L.stream, uint32_t(N), Rx0, Rx1, Ry0, Ry1, C0, C1, xhat, yhat, out);
+      return hipGetLastError();
+    };
+    // a few graphs: rows of the tile to more CUs (one graph of 140 nodes is 9
+    // workgroups of 16 rows, a chain of staging and output loads each)
+    if (graphs * ((N + TI - 1) / TI) < size_t(L.num_cu)) return go(std::integral_constant<int, 2>{});
+    return go(std::integral_constant<int, TI>{});
   }
-  const int grid = grid_for(k_mul_eval_sum<T>, block, lay.nz, L.num_cu);
+  const int grid = grid_for(k_mul_eval_sum<T>, block, (lay.nz + kMulUnroll - 1) / kMulUnroll, L.num_cu);
   hipLaunchKernelGGL((k_mul_eval_sum<T>), dim3(grid), dim3(block), 0, L.stream, lay.nz, Rx0, Rx1, Ry0, Ry1, C0, C1, map,
                      xhat, yhat, out);
   return hipGetLastError();
@@ -813,11 +838,69 @@ hipError_t launch_lut8_keygen(const Launch &L, const Lut8Layout &lay, uint64_t s
 
 // Phase 1: full-domain expansion of the 8-bit DPF (1 tree level + two 128-bit
 // leaves) and the signed inner product with the public table rotated by x^.
+// Sum of table[j] over the 256 positions j with u[(xh - j) mod 256] set.  The bits
+// are reversed and rotated by the lane's x^, so that every lane adds the same
+// table entry at a time, read by all lanes at one address of the LDS copy tab,
+// under a mask of its own bit: three VALU instructions an entry (walking the set
+// bits took a divergent loop of some 170 rounds of conflicting table reads: the
+// phase 148 us beside two other groups' work at 47 k elements, now 62 with the
+// whole gate).
+template <typename T>
+__device__ __forceinline__ T lut8_sum(uint4 lo, uint4 hi, uint32_t xh, const T *tab) {
+  uint32_t w[8] = {__brev(hi.w), __brev(hi.z), __brev(hi.y), __brev(hi.x),
+                   __brev(lo.w), __brev(lo.z), __brev(lo.y), __brev(lo.x)};
+  const uint32_t s = (255u - xh) & 255u;  // w rotated right by s: bit j is u[xh - j]
+#pragma unroll
+  for (int b = 1; b < 8; b *= 2) {
+    uint32_t v[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] = (s & (32u * uint32_t(b))) ? w[(q + b) & 7] : w[q];
+#pragma unroll
+    for (int q = 0; q < 8; q++) w[q] = v[q];
+  }
+  T acc = 0;
+  constexpr int W = 16 / int(sizeof(T));  // entries per 16-byte read
+#pragma unroll 1
+  for (int q = 0; q < 8; q++) {
+    const uint32_t bits = __builtin_amdgcn_alignbit(w[1], w[0], s & 31u);
+    const uint32_t w0 = w[0];
+#pragma unroll
+    for (int k = 0; k < 7; k++) w[k] = w[k + 1];
+    w[7] = w0;
+    T t[32];
+#pragma unroll
+    for (int g = 0; g < 32 / W; g++)
+      __builtin_memcpy(t + g * W, reinterpret_cast<const uint4 *>(tab) + q * (32 / W) + g, 16);
+#pragma unroll
+    for (int b = 0; b < 32; b++) acc += T(std::make_signed_t<T>(int32_t(bit_mask(bits, b)))) & t[b];
+  }
+  return acc;
+}
+
+// Party p's message of the first round: +-sum plus its share of the mask.
+template <typename T, class Aes>
+__device__ __forceinline__ T lut8_message(const Aes &aes, const Lut8Layout &lay, int p, const uint8_t *K,
+                                          const uint8_t *KC, size_t i, uint32_t xh, const T *tab) {
+  const uint4 s = reinterpret_cast<const uint4 *>(K + lay.dpf.off_root)[i];
+  // correction and leaf words are common to both parties' keys
+  const uint4 cw = reinterpret_cast<const uint4 *>(KC + lay.dpf.off_cw)[i];
+  const uint4 leaf = reinterpret_cast<const uint4 *>(KC + lay.dpf.off_leaf)[i];
+  const T rv = reinterpret_cast<const T *>(K + lay.off_rv)[i];
+  const uint32_t t = bit_mask(s.x, 0);
+  const uint4 sl = xor_and4(aes.hash(s, c_rkH), cw, t);
+  const uint4 sr = xor4(sl, s);
+  const uint32_t tl = bit_mask(sl.x, 0);
+  uint4 L0, L1;
+  hash_pair(aes, sl, sr, c_rkL, &L0, &L1);
+  const T acc = lut8_sum(xor_and4(L0, leaf, tl), xor_and4(L1, leaf, tl ^ t), xh, tab);
+  return (p ? T(0) - acc : acc) + rv;
+}
+
 template <typename T, int NT, int REP>
 __global__ void k_lut8_phase1(Lut8Layout lay, const uint8_t *k0, const uint8_t *k1,
                               const T *table, const T *xhat, T *msg0, T *msg1, int pbase) {
   __shared__ __align__(16) uint32_t lds[AesLds<NT, REP>::kWords];
-  __shared__ T tab[256];
+  __shared__ __align__(16) T tab[256];
   for (int k = threadIdx.x; k < 256; k += blockDim.x) tab[k] = table[k];
   AesLds<NT, REP>::fill(lds);
   AesLds<NT, REP> aes(lds);
@@ -825,32 +908,56 @@ __global__ void k_lut8_phase1(Lut8Layout lay, const uint8_t *k0, const uint8_t *
   const uint8_t *K = p ? k1 : k0;
   T *msg = p ? msg1 : msg0;
   const size_t N = lay.dpf.N;
-  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < N; i += size_t(gridDim.x) * blockDim.x) {
-    const uint4 s = reinterpret_cast<const uint4 *>(K + lay.dpf.off_root)[i];
-    // correction and leaf words are common to both parties: read party 0's
-    const uint4 cw = reinterpret_cast<const uint4 *>(k0 + lay.dpf.off_cw)[i];
-    const uint4 leaf = reinterpret_cast<const uint4 *>(k0 + lay.dpf.off_leaf)[i];
-    const uint32_t t = s.x & 1u;
-    const uint4 sl = xor4(aes.hash(s, c_rkH), and4(cw, 0u - t));
-    const uint4 sr = xor4(sl, s);
-    const uint32_t tl = sl.x & 1u, tr = tl ^ t;
-    const uint4 L0 = xor4(aes.hash(sl, c_rkL), and4(leaf, 0u - tl));
-    const uint4 L1 = xor4(aes.hash(sr, c_rkL), and4(leaf, 0u - tr));
-    const uint32_t w[8] = {L0.x, L0.y, L0.z, L0.w, L1.x, L1.y, L1.z, L1.w};
-    const uint32_t xh = uint32_t(xhat[i]) & 255u;
-    T acc = 0;
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      uint32_t bits = w[q];
-      while (bits) {
-        const int b = __ffs(bits) - 1;
-        bits &= bits - 1;
-        acc += tab[(xh - uint32_t(q * 32 + b)) & 255u];
-      }
-    }
-    if (p == 1) acc = T(0) - acc;
-    msg[i] = acc + reinterpret_cast<const T *>(K + lay.off_rv)[i];
+  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < N; i += size_t(gridDim.x) * blockDim.x)
+    msg[i] = lut8_message(aes, lay, p, K, k0, i, uint32_t(xhat[i]) & 255u, tab);
+}
+
+// The whole gate for both parties: lanes 2e and 2e + 1 are the parties of an
+// element and exchange their two messages through DPP (lane ^ 1).  One launch
+// instead of four; at 140 elements (one molecule) the gate took 32 us, mostly one
+// thread's walk over 128 set bits and three more launches.
+__device__ __forceinline__ uint32_t from_pair(uint32_t v) {
+  return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0xb1, 0xf, 0xf, false));  // lanes 1,0,3,2
+}
+__device__ __forceinline__ uint64_t from_pair(uint64_t v) {
+  return uint64_t(from_pair(uint32_t(v))) | (uint64_t(from_pair(uint32_t(v >> 32))) << 32);
+}
+template <typename T, int NT, int REP>
+__global__ void k_lut8_sum(Lut8Layout lay, const uint8_t *k0, const uint8_t *k1, const T *table, const T *xhat,
+                           T *out) {
+  __shared__ __align__(16) uint32_t lds[AesLds<NT, REP>::kWords];
+  __shared__ __align__(16) T tab[256];
+  for (int k = threadIdx.x; k < 256; k += blockDim.x) tab[k] = table[k];
+  AesLds<NT, REP>::fill(lds);
+  AesLds<NT, REP> aes(lds);
+  const int p = int(threadIdx.x & 1u);
+  const uint8_t *K = p ? k1 : k0;
+  const size_t N = lay.dpf.N, stride = size_t(gridDim.x) * blockDim.x / 2;
+  const size_t rounds = (N + stride - 1) / stride;  // whole waves: both lanes of a pair run to the end
+  size_t i = (size_t(blockIdx.x) * blockDim.x + threadIdx.x) / 2;
+  for (size_t r = 0; r < rounds; r++, i += stride) {
+    const size_t e = i < N ? i : N - 1;
+    // loaded ahead of the hashes
+    const T sig = reinterpret_cast<const T *>(K + lay.off_sig)[e], c = reinterpret_cast<const T *>(K + lay.off_c)[e];
+    const T m = lut8_message(aes, lay, p, K, k0, e, uint32_t(xhat[e]) & 255u, tab);
+    const T vh = m + from_pair(m);  // exchange 1: the revealed masked sum
+    const T z = vh * sig + c;
+    const T y = z + from_pair(z);  // exchange 2: the revealed output
+    if (p == 0 && i < N) out[i] = y;
   }
+}
+template <typename T>
+hipError_t launch_lut8_sum(const Launch &L, const Lut8Layout &lay, const uint8_t *k0, const uint8_t *k1,
+                           const T *table, const T *xhat, T *out) {
+  if (lay.dpf.N == 0) return hipSuccess;
+  return with_variant(L, [&](auto v) {
+    constexpr int NT = decltype(v)::nt, REP = decltype(v)::rep;
+    // few elements: one wave of them per workgroup in 256 threads that fill its table
+    const int block = L.aes_block > 0 ? L.aes_block : lay.dpf.N < 128 * size_t(L.num_cu) ? 256 : variant_block(L);
+    const int grid = grid_for(k_lut8_sum<T, NT, REP>, block, 2 * lay.dpf.N, L.num_cu);
+    hipLaunchKernelGGL((k_lut8_sum<T, NT, REP>), dim3(grid), dim3(block), 0, L.stream, lay, k0, k1, table, xhat, out);
+    return hipGetLastError();
+  });
 }
 
 template <typename T>
@@ -1113,6 +1220,8 @@ hipError_t launch_rowsum(const Launch &L, size_t rows, int len, const T *a, T *o
                                             uint8_t *, uint8_t *);                                                    \
   template hipError_t launch_lut8_phase1<T>(const Launch &, const Lut8Layout &, const uint8_t *, const uint8_t *,     \
                                             const T *, const T *, T *, T *);                                          \
+  template hipError_t launch_lut8_sum<T>(const Launch &, const Lut8Layout &, const uint8_t *, const uint8_t *,       \
+                                         const T *, const T *, T *);                                                 \
   template hipError_t launch_lut8_phase2<T>(const Launch &, const Lut8Layout &, const uint8_t *, const uint8_t *,     \
                                             const T *, T *, T *);                                                     \
   template hipError_t launch_split<T>(const Launch &, uint64_t, uint32_t, uint32_t, size_t, const T *, T *, T *,      \

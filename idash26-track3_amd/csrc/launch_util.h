@@ -47,6 +47,25 @@ inline int grid_for(K kernel, int block, size_t n, int num_cu) {
 }
 
 
+// True where n1 bytes at p and n2 bytes at q do not overlap.
+inline bool bytes_apart(const void *p, size_t n1, const void *q, size_t n2) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+  return a + n1 <= b || b + n2 <= a;
+}
+
+// A value in uniform memory that the kernel does not write (its arguments, a
+// table), read into scalar registers.
+using ConstWord = const __attribute__((address_space(4))) uint32_t;
+template <class S>
+__device__ __forceinline__ S load_uniform(ConstWord *p) {
+  uint32_t w[sizeof(S) / 4];
+#pragma unroll
+  for (size_t k = 0; k < sizeof(S) / 4; k++) w[k] = p[k];
+  S s;
+  __builtin_memcpy(&s, w, sizeof(S));
+  return s;
+}
+
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
 
 template <typename T>

@@ -441,12 +441,9 @@ struct Runner {
       leave(end);
       return hipSuccess;
     }
-    TRY(launch_lut8_phase1<T>(L, lay, kv.k[0], kv.k[1], table, x, ws.m0.p, ws.m1.p));
     ctr.msg(n, bw);
-    TRY(launch_reconstruct<T>(L, n, ws.m0.p, ws.m1.p, vh));
-    TRY(launch_lut8_phase2<T>(L, lay, kv.k[0], kv.k[1], vh, ws.m0.p, ws.m1.p));
     ctr.msg(n, bw);
-    TRY(launch_reconstruct<T>(L, n, ws.m0.p, ws.m1.p, out));
+    TRY(launch_lut8_sum<T>(L, lay, kv.k[0], kv.k[1], table, x, out));
     leave(end);
     return hipSuccess;
   }
