@@ -254,14 +254,24 @@ struct AesPerm2 {
   const char *base;
   uint32_t lane4;  // (lane * 4) mod 128
 
-  // 16-byte stores: entry x is 8 stores of T0[x], then 8 of T1[x]
+  // Entry x is 8 16-byte words of T0[x], then 8 of T1[x]; a thread writes one of
+  // the two halves of an entry, starting at word x mod 8, so that 16 lanes' stores
+  // cover the 64 banks.  The reads of T0 go out together: a loop of one read per
+  // store spends a memory latency per iteration, and this is what a launch of few
+  // elements starts with (1024 truncations 33.7 -> 32.6 us, a forward of one
+  // sample 501 -> 487 us).
   __device__ static void fill(uint32_t *lds) {
     uint4 *l4 = reinterpret_cast<uint4 *>(lds);
-    for (int q = threadIdx.x; q < kWords / 4; q += blockDim.x) {
-      const uint32_t t = c_T0.v[q >> 4];
-      const uint32_t v = (q & 8) ? rotl32(t, 8) : t;
-      l4[q] = make_uint4(v, v, v, v);
-    }
+    const uint32_t nt = blockDim.x, q0 = threadIdx.x, q1 = q0 + nt;
+    const uint32_t w0 = c_T0.v[(q0 >> 1) & 255u], w1 = nt < 512 ? c_T0.v[(q1 >> 1) & 255u] : 0u;
+    auto half = [&](uint32_t q, uint32_t t) {
+      const uint32_t v = (q & 1u) ? rotl32(t, 8) : t;
+#pragma unroll
+      for (uint32_t k = 0; k < 8; k++) l4[8 * q + ((k + (q >> 1)) & 7u)] = make_uint4(v, v, v, v);
+    };
+    if (q0 < 512) half(q0, w0);
+    if (q1 < 512) half(q1, w1);
+    for (uint32_t q = q1 + nt; q < 512; q += nt) half(q, c_T0.v[q >> 1]);
     __syncthreads();
   }
 
