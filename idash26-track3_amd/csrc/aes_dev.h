@@ -260,17 +260,26 @@ struct AesPerm2 {
   // store spends a memory latency per iteration, and this is what a launch of few
   // elements starts with (1024 truncations 33.7 -> 32.6 us, a forward of one
   // sample 501 -> 487 us).
-  __device__ static void fill(uint32_t *lds) {
+  // fill_words() issues those reads, so that a kernel can put its own behind them
+  // before it waits.
+  struct FillWords {
+    uint32_t w0, w1;
+  };
+  __device__ static FillWords fill_words() {
+    const uint32_t nt = blockDim.x, q0 = threadIdx.x, q1 = q0 + nt;
+    return {c_T0.v[(q0 >> 1) & 255u], nt < 512 ? c_T0.v[(q1 >> 1) & 255u] : 0u};
+  }
+  __device__ static void fill(uint32_t *lds) { fill(lds, fill_words()); }
+  __device__ static void fill(uint32_t *lds, const FillWords &w) {
     uint4 *l4 = reinterpret_cast<uint4 *>(lds);
     const uint32_t nt = blockDim.x, q0 = threadIdx.x, q1 = q0 + nt;
-    const uint32_t w0 = c_T0.v[(q0 >> 1) & 255u], w1 = nt < 512 ? c_T0.v[(q1 >> 1) & 255u] : 0u;
     auto half = [&](uint32_t q, uint32_t t) {
       const uint32_t v = (q & 1u) ? rotl32(t, 8) : t;
 #pragma unroll
       for (uint32_t k = 0; k < 8; k++) l4[8 * q + ((k + (q >> 1)) & 7u)] = make_uint4(v, v, v, v);
     };
-    if (q0 < 512) half(q0, w0);
-    if (q1 < 512) half(q1, w1);
+    if (q0 < 512) half(q0, w.w0);
+    if (q1 < 512) half(q1, w.w1);
     for (uint32_t q = q1 + nt; q < 512; q += nt) half(q, c_T0.v[q >> 1]);
     __syncthreads();
   }

@@ -420,33 +420,42 @@ template <typename T, bool TWO, bool POOL>
 __device__ __forceinline__ void tr_eval_tiles_quad(const TrArgs<T> &a, const TrArgs<T> &a2, const TrPool<T> &q) {
   __shared__ __align__(16) uint32_t lds[AesPerm2::kWords];
   __shared__ TrXchg<T> x;
-  AesPerm2::fill(lds);
   const AesPerm2 tab(lds);
   const AesQuad aes(tab);
-  const AesQuad::Keys kH = aes.keys(c_rkH), kL = aes.keys(c_rkL);
   const int hq = int(blockDim.x) / 2, h = hq / 4;
   const int p = int(threadIdx.x) >= hq ? 1 : 0;
   const int lt = int(threadIdx.x) - p * hq;  // thread of the party's half
   const int e = lt >> 2, wv = lt >> 6;
   const uint8_t *K = p ? a.k1 : a.k0, *KC = a.k0;
   const size_t stride = size_t(gridDim.x) * size_t(h);
-  for (size_t base = size_t(blockIdx.x) * h; base < a.N; base += stride) {
-    const size_t i = base + size_t(e);
-    const bool in = i < a.N;
-    T xin = 0, v0 = 0;
-    uint32_t o = 0;
-    QuadKeys<T> qk, qk2;
-    if (in) {
-      qk = quad_keys(a, aes.j, K, KC, i);
-      if constexpr (POOL) {
-        const uint32_t s0 = pool_src(q, uint32_t(i), &o);
-        v0 = q.v[s0];
-        xin = q.v[s0 + q.C] - v0;
-      } else {
-        xin = a.xhat[i];
-      }
-      if constexpr (TWO) qk2 = quad_keys(a2, aes.j, K, KC, i);
+  // a tile's input and key words; the first tile's, and the round keys, are on
+  // their way while the AES table is written (behind the table's own reads, which
+  // return first; a forward of one sample 487 -> 468 us)
+  size_t i = 0;
+  bool in = false;
+  T xin = 0, v0 = 0;
+  uint32_t o = 0;
+  QuadKeys<T> qk, qk2;
+  auto load = [&](size_t base) {
+    i = base + size_t(e);
+    in = i < a.N;
+    if (!in) return;
+    if constexpr (POOL) {
+      const uint32_t s0 = pool_src(q, uint32_t(i), &o);
+      v0 = q.v[s0];
+      xin = q.v[s0 + q.C] - v0;
+    } else {
+      xin = a.xhat[i];
     }
+    qk = quad_keys(a, aes.j, K, KC, i);
+    if constexpr (TWO) qk2 = quad_keys(a2, aes.j, K, KC, i);
+  };
+  size_t base = size_t(blockIdx.x) * h;
+  const AesPerm2::FillWords fw = AesPerm2::fill_words();
+  const AesQuad::Keys kH = aes.keys(c_rkH), kL = aes.keys(c_rkL);
+  load(base);
+  AesPerm2::fill(lds, fw);
+  while (base < a.N) {
     T y = tr_tile_quad(aes, kH, kL, a, x, p, e, wv, qk, KC, i, in, xin);
     if constexpr (TWO) y = tr_tile_quad(aes, kH, kL, a2, x, p, e, wv, qk2, KC, i, in, y);
     if (p == 0 && in && (lt & 3) == 0) {
@@ -455,6 +464,8 @@ __device__ __forceinline__ void tr_eval_tiles_quad(const TrArgs<T> &a, const TrA
       else
         a.out[i] = y;
     }
+    base += stride;
+    load(base);
   }
   if constexpr (POOL) pool_carry(q);
 }
@@ -504,7 +515,7 @@ __global__ void k_tr_eval_pool_tail_q(TrTail<T> t) {
   __shared__ __align__(16) uint32_t lds[AesPerm2::kWords];
   __shared__ TrXchg<T> x;
   extern __shared__ __align__(16) unsigned char tail_lds[];
-  AesPerm2::fill(lds);
+  const AesPerm2::FillWords fw = AesPerm2::fill_words();
   const AesPerm2 tab(lds);
   const AesQuad aes(tab);
   const AesQuad::Keys kH = aes.keys(c_rkH), kL = aes.keys(c_rkL);
@@ -521,7 +532,7 @@ __global__ void k_tr_eval_pool_tail_q(TrTail<T> t) {
     const int cc = k / R0, r = k - cc * R0, g = g0 + cc, b = g / C, c = g - b * C;
     vin[k] = t.v[(size_t(b) * R0 + r) * C + c];
   }
-  __syncthreads();
+  AesPerm2::fill(lds, fw);  // ends with the barrier that vin waits for
   int R = R0;
   for (int l = 0; l < t.nlev; l++) {
     TrArgs<T> a = t.a;
