@@ -183,8 +183,13 @@ def to_dev(a):
 
 
 def empty_dev(nbytes):
+    """Zeroed device bytes, zeroed when this returns: the library works on a
+    stream that is not ordered with torch's, so a fill still pending there could
+    land on top of its results."""
     torch = _torch()
-    return torch.zeros(max(int(nbytes), 1), dtype=torch.uint8, device="cuda")
+    t = torch.zeros(max(int(nbytes), 1), dtype=torch.uint8, device="cuda")
+    torch.cuda.current_stream().synchronize()
+    return t
 
 
 def from_dev(t, dtype, count=None):

@@ -16,6 +16,16 @@
  * elements (n = 0; nz = 0 for mpcx_mul_eval, rows = 0 for mpcx_ring_lincomb)
  * returns MPCX_OK without reading its pointers or counting an exchange; matrix
  * dimensions (B, N, C, nb, M, K) must be at least 1.
+ *
+ * A call reads and writes its device buffers on the context's stream, which is
+ * non-blocking (mpcx_set_stream: another one): work of other streams on these
+ * buffers, the null stream's fills and copies included, has to be done, or
+ * ordered before that stream, when the call is made.  mpcx_prg_hash, mpcx_prf,
+ * mpcx_dcf_*, mpcx_tr_keygen, mpcx_mul_keygen, mpcx_lut8_keygen,
+ * mpcx_reveal_keygen, mpcx_ring_gemm, mpcx_ring_lincomb,
+ * mpcx_maxpool_eval_noalloc and, with mpcx_set_party_sync(ctx, 0),
+ * mpcx_party_* return with their work enqueued there: their buffers stay in
+ * use until the stream has reached it.
  */
 #ifndef MPCX_H
 #define MPCX_H
