@@ -305,6 +305,7 @@ class Ctx:
         dr = to_dev(np.ascontiguousarray(rbit, np.uint8)) if rbit is not None else None
         self.check(self.lib.mpcx_dcf_keygen(self.h, m, n, dptr(da), dptr(dr), seed, gate, dptr(k0), dptr(k1)),
                    "dcf_keygen")
+        self.sync()  # the call is only enqueued: alpha and rbit are read until then
         return k0, k1
 
     def dcf_eval(self, party, m, key, x):

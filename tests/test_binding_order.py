@@ -71,8 +71,9 @@ def _torch_on(st):
 
 
 # entry points that return with their work enqueued
-ENQUEUES = {"mpcx_prg_hash", "mpcx_prf", "mpcx_dcf_keygen", "mpcx_dcf_eval", "mpcx_dcf_eval_ring", "mpcx_tr_keygen", "mpcx_mul_keygen",
-            "mpcx_lut8_keygen", "mpcx_reveal_keygen", "mpcx_ring_gemm", "mpcx_maxpool_eval_noalloc"}
+ENQUEUES = {"mpcx_prg_hash", "mpcx_prf", "mpcx_dcf_keygen", "mpcx_dcf_eval", "mpcx_dcf_eval_ring",
+            "mpcx_tr_keygen", "mpcx_mul_keygen", "mpcx_lut8_keygen", "mpcx_reveal_keygen", "mpcx_ring_gemm",
+            "mpcx_maxpool_eval_noalloc"}
 
 
 class Lib:
@@ -108,6 +109,7 @@ PEER = types.SimpleNamespace(h=ctypes.c_void_p(0))
 CALLS = {
     "prg_hash": lambda c: c.prg_hash(np.zeros((2, 4), np.uint32)),
     "prf": lambda c: c.prf(1, 2, 3, 4),
+    "dcf_keygen": lambda c: c.dcf_keygen(12, V, np.zeros(8, np.uint8)),
     "dcf_eval": lambda c: c.dcf_eval(0, 12, K, V),
     "dcf_eval_ring": lambda c: c.dcf_eval_ring(0, 12, K, V, np.zeros(1, np.uint32)),
     "tr_keygen": lambda c: c.tr_keygen(1, V),
