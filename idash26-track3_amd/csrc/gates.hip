@@ -673,14 +673,6 @@ struct TrGenArgs {
   size_t tiles = 0;
 };
 
-// Hides where a pointer to uniform memory comes from, so that what is read
-// through it is read there: round keys of three keys at once would not fit the
-// scalar registers and be spilled to vector lanes.
-__device__ __forceinline__ ConstWord *fresh(ConstWord *p) {
-  asm volatile("" : "+s"(p));
-  return p;
-}
-
 // The dealer's entry c of a gate's G table before it is split: r the input mask,
 // rho its sign bit, rout the output mask, ba and bd the DCF output masks.
 template <typename T>

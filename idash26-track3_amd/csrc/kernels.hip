@@ -305,14 +305,21 @@ __global__ void k_split(AesRK kd, uint32_t gate, uint32_t field, size_t n, const
   AesLds<NT, REP>::fill(lds);
   AesLds<NT, REP> aes(lds);
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) {
-    T val;
-    if (v) {
-      val = v[i];
-    } else {  // fresh reveal mask
-      val = ring_of<T>(aes.prf(kd, gate, F_RIN, i));
-      mask_out[i] = val;
+    T val, s0;
+    if (sizeof(T) == 8 && !v) {  // its blocks side by side (10^6 words 28.2 against 28.9 us)
+      uint4 b0, b1;
+      prf2(aes, kd, gate, F_RIN, field, i, &b0, &b1);
+      mask_out[i] = val = ring_of<T>(b0);
+      s0 = ring_of<T>(b1);
+    } else {  // 32-bit masks one after the other (26.3 against 26.9)
+      if (v) {
+        val = v[i];
+      } else {  // fresh reveal mask
+        val = ring_of<T>(aes.prf(kd, gate, F_RIN, i));
+        mask_out[i] = val;
+      }
+      s0 = ring_of<T>(aes.prf(kd, gate, field, i));
     }
-    const T s0 = ring_of<T>(aes.prf(kd, gate, field, i));
     p0[i] = s0;
     p1[i] = val - s0;
     if (copy0) copy0[i] = s0;
@@ -786,6 +793,9 @@ hipError_t launch_mul_eval_sum(const Launch &L, const MulLayout &lay, const uint
 // ---------------------------------------------------------------------------
 // 8-bit DPF lookup table
 // ---------------------------------------------------------------------------
+// The round keys are read again after the walk, where 44 of them held across it
+// spilled 23 vector registers, and the PRF blocks go two by two: 10^6 keys 130 us
+// against 136, 1000 23.3 against 25.0.
 template <typename T, int NT, int REP>
 __global__ void k_lut8_keygen(AesRK kd, uint32_t gate, Lut8Layout lay, const T *in_mask,
                               T *out_mask, uint8_t *k0, uint8_t *k1) {
@@ -793,12 +803,13 @@ __global__ void k_lut8_keygen(AesRK kd, uint32_t gate, Lut8Layout lay, const T *
   AesLds<NT, REP>::fill(lds);
   AesLds<NT, REP> aes(lds);
   const size_t N = lay.dpf.N;
+  ConstWord *args = (ConstWord *)__builtin_amdgcn_kernarg_segment_ptr();  // kd
   for (size_t base = size_t(blockIdx.x) * blockDim.x; base < N; base += size_t(gridDim.x) * blockDim.x) {
     const size_t i = base + threadIdx.x;
     if (i >= N) break;
     const uint32_t alpha = uint32_t(in_mask[i]) & 255u;
     uint4 root0, root1;
-    dealer_roots(aes, kd, gate, F_DCFA, i, &root0, &root1);
+    dealer_roots(aes, load_uniform<AesRK>(fresh(args)), gate, F_DCFA, i, &root0, &root1);
     const DcfGenOut g = dcf_gen_walk(aes, root0, root1, lay.dpf, alpha, base, threadIdx.x, k0, k1);
     const uint4 lb = xor4(aes.hash(g.s0, c_rkL), and4(g.leafcw, g.t0));
     const uint32_t pos = uint32_t(alpha & 127u);
@@ -806,13 +817,15 @@ __global__ void k_lut8_keygen(AesRK kd, uint32_t gate, Lut8Layout lay, const T *
     const uint32_t word = wsel == 0 ? lb.x : wsel == 1 ? lb.y : wsel == 2 ? lb.z : lb.w;
     const uint32_t u0 = (word >> (pos & 31u)) & 1u;
     const T sigma = u0 ? T(1) : T(0) - T(1);
-    const T rv = ring_of<T>(aes.prf(kd, gate, F_LUTV, i));
-    const T rout = ring_of<T>(aes.prf(kd, gate, F_ROUT, i));
+    uint4 b0, b1;
+    const AesRK k = load_uniform<AesRK>(fresh(args));
+    prf2(aes, k, gate, F_LUTV, F_ROUT, i, &b0, &b1);
+    const T rv = ring_of<T>(b0), rout = ring_of<T>(b1);
     out_mask[i] = rout;
     const T C = rout - sigma * rv;
-    const T v0 = ring_of<T>(aes.prf(kd, gate, F_SPLIT + 0, i));
-    const T s0 = ring_of<T>(aes.prf(kd, gate, F_SPLIT + 1, i));
-    const T c0 = ring_of<T>(aes.prf(kd, gate, F_SPLIT + 2, i));
+    prf2(aes, k, gate, F_SPLIT + 0, F_SPLIT + 1, i, &b0, &b1);
+    const T v0 = ring_of<T>(b0), s0 = ring_of<T>(b1);
+    const T c0 = ring_of<T>(aes.prf(k, gate, F_SPLIT + 2, i));
     reinterpret_cast<T *>(k0 + lay.off_rv)[i] = v0;
     reinterpret_cast<T *>(k1 + lay.off_rv)[i] = rv - v0;
     reinterpret_cast<T *>(k0 + lay.off_sig)[i] = s0;

@@ -66,6 +66,14 @@ __device__ __forceinline__ S load_uniform(ConstWord *p) {
   return s;
 }
 
+// Hides where a pointer to uniform memory comes from, so that what is read
+// through it is read there: round keys of three keys at once would not fit the
+// scalar registers and be spilled to vector lanes.
+__device__ __forceinline__ ConstWord *fresh(ConstWord *p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
 
 template <typename T>
