@@ -391,8 +391,10 @@ struct AesPerm2 {
   // of the next ones are on their way: with a single chain a phase forms all four
   // columns and then waits for all reads.  25 hashes one after another take 34
   // against 41 us with one wave per SIMD, 42-45 in both orders with 1.5 and two and
-  // 72-73 with four.  PRF blocks take this order: 10^6 Beaver keys 52.9 us against
-  // 55.7 in phases, 10^6 blocks alone 17.9 against 18.3.
+  // 72-73 with four; but the order needs more registers, and one held to 64 of them
+  // keeps few reads in flight (146 against 103 us for 64-bit ReLUs of 160 elements
+  // per CU).  So PRF blocks and the gates of small workgroups (AesPerm2Few) take
+  // this order, the other walks the phases.
   __device__ __forceinline__ uint32_t col(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t k) const {
     const uint32_t h = xor3(t0<2>(c), t1<3>(d), (k << 16) | (k >> 16));
     return xor3(t0<0>(a), t1<1>(b), __builtin_amdgcn_alignbit(h, h, 16));
@@ -450,6 +452,16 @@ struct AesPerm2 {
     b.z = field;
     b.w = gate;
     return enc(b, kd);
+  }
+};
+
+// AesPerm2 with single hashes in the scheduler's order (AesPerm2::block).
+struct AesPerm2Few : AesPerm2 {
+  using AesPerm2::AesPerm2;
+  __device__ __forceinline__ uint4 hash(uint4 s, const AesRK &rk) const {
+    const uint4 o = block(hash_in(s, rk), rk);
+    return make_uint4(xor3(o.x, rk.w[40], s.z), xor3(o.y, rk.w[41], s.w), xor3(o.z, rk.w[42], s.z) ^ s.x,
+                      xor3(o.w, rk.w[43], s.w) ^ s.y);
   }
 };
 

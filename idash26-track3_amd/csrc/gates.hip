@@ -224,12 +224,12 @@ __device__ __forceinline__ T tr_tile(const Aes &aes, const TrArgs<T> &a, TrXchg<
 // The tiles of one launch: gate a on x^, then (TWO) gate a2 on a's revealed
 // output, which both parties hold once it is revealed; party 0's threads write
 // the last gate's revealed output.
-template <typename T, int NT, int REP, bool TWO, bool POOL>
+template <typename T, class Aes, bool TWO, bool POOL>
 __device__ __forceinline__ void tr_eval_tiles(const TrArgs<T> &a, const TrArgs<T> &a2, const TrPool<T> &q) {
-  __shared__ __align__(16) uint32_t lds[AesLds<NT, REP>::kWords];
+  __shared__ __align__(16) uint32_t lds[Aes::kWords];
   __shared__ TrXchg<T> x;
-  AesLds<NT, REP>::fill(lds);
-  AesLds<NT, REP> aes(lds);
+  Aes::fill(lds);
+  const Aes aes(lds);
   const int h = int(blockDim.x) / 2;
   // a party's half is whole waves, so the party is uniform over a wave
   const int p = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >= h ? 1 : 0);
@@ -570,30 +570,41 @@ __global__ void k_tr_eval_pool_tail_q(TrTail<T> t) {
   for (int k = int(threadIdx.x); k < nc; k += int(blockDim.x)) t.out[g0 + k] = vin[k * R0];
 }
 
-// 64 registers, so that two 1024-thread workgroups fit a CU where a launch takes
-// them (the rounds' reads go out in phases, AesPerm2, so fewer registers cost no
-// order of loads).
-template <typename T, int NT, int REP, int TAG>
-__global__ void __launch_bounds__(1024, 8) k_tr_eval(TrArgs<T> a) {
+// The one-lane kernels' instances.  kFew: a CU has few waves (tr_few), whose walks
+// take the scheduler's order of reads (AesPerm2Few); kMid: the phases; kWide: 1024
+// threads in 64 registers, so that two such workgroups fit a CU (2 spilled, 8 in
+// Z_2^64: outside the level loops, but each a memory latency, 0.5 us, in a launch of
+// few waves).  All launches in the 64 registers and the phases, against now: RELUs
+// of 79 elements per CU 57.1 -> 46.6 us (Z_2^64 107.6 -> 85.9), of 256 57.5 -> 55.6
+// (108.2 -> 105.2), 6-call TRMODs of 129 to 512 26.5-34.1 -> 25.9-33.3.
+enum { kFew, kMid, kWide };
+constexpr int kFewThreads = 512;
+constexpr int inst_threads(int I) { return I == kFew ? kFewThreads : 1024; }
+constexpr int inst_waves(int I) { return I == kFew ? 5 : I == kMid ? 4 : 8; }
+template <int NT, int REP, int I>
+using TrAes = std::conditional_t<I == kFew, AesPerm2Few, AesLds<NT, REP>>;
+
+template <typename T, int NT, int REP, int I, int TAG>
+__global__ void __launch_bounds__(inst_threads(I), inst_waves(I)) k_tr_eval(TrArgs<T> a) {
   if (a.prio) __builtin_amdgcn_s_setprio(2);
-  tr_eval_tiles<T, NT, REP, false, false>(a, a, TrPool<T>{});
+  tr_eval_tiles<T, TrAes<NT, REP, I>, false, false>(a, a, TrPool<T>{});
 }
 
 // The max-pool form (TrPool) of k_tr_eval.
-template <typename T, int NT, int REP, int TAG>
-__global__ void k_tr_eval_pool(TrArgs<T> a, TrPool<T> q) {
+template <typename T, int NT, int REP, int I, int TAG>
+__global__ void __launch_bounds__(inst_threads(I), inst_waves(I)) k_tr_eval_pool(TrArgs<T> a, TrPool<T> q) {
   if (a.prio) __builtin_amdgcn_s_setprio(2);
-  tr_eval_tiles<T, NT, REP, false, true>(a, a, q);
+  tr_eval_tiles<T, TrAes<NT, REP, I>, false, true>(a, a, q);
 }
 
 // Two gates of one element count in one launch (a truncation and its extension):
 // the second gate's masked input is the first's revealed output, element by
 // element, so no workgroup waits on another and the intermediate stays in
 // registers.  Output in a.out.
-template <typename T, int NT, int REP, int TAG>
-__global__ void k_tr_eval2(TrArgs<T> a, TrArgs<T> a2) {
+template <typename T, int NT, int REP, int I, int TAG>
+__global__ void __launch_bounds__(inst_threads(I), inst_waves(I)) k_tr_eval2(TrArgs<T> a, TrArgs<T> a2) {
   if (a.prio) __builtin_amdgcn_s_setprio(2);
-  tr_eval_tiles<T, NT, REP, true, false>(a, a2, TrPool<T>{});
+  tr_eval_tiles<T, TrAes<NT, REP, I>, true, false>(a, a2, TrPool<T>{});
 }
 
 // Both-party forms: one thread per element for both parties.
@@ -1050,6 +1061,39 @@ static void tr_both_launch(const Launch &L, const TrArgs<T> &a, const TrPool<T> 
     hipLaunchKernelGGL((k_tr_eval_b<T, NT, REP, W, 0>), dim3(grid), dim3(block), 0, L.stream, a);
 }
 
+template <typename T, int NT, int REP, int I>
+static void tr_one_launch(const Launch &L, const TrArgs<T> &a, int block) {
+  const int grid = grid_for(k_tr_eval<T, NT, REP, I, 0>, block, 2 * a.N, L.num_cu);
+  if (L.profiled)
+    hipLaunchKernelGGL((k_tr_eval<T, NT, REP, I, 1>), dim3(grid), dim3(block), 0, L.stream, a);
+  else
+    hipLaunchKernelGGL((k_tr_eval<T, NT, REP, I, 0>), dim3(grid), dim3(block), 0, L.stream, a);
+}
+template <typename T, int NT, int REP, int I>
+static void tr_pool_launch(const Launch &L, const TrArgs<T> &a, const TrPool<T> &q, int block) {
+  const int grid = grid_for(k_tr_eval_pool<T, NT, REP, I, 0>, block, 2 * a.N, L.num_cu);
+  if (L.profiled)
+    hipLaunchKernelGGL((k_tr_eval_pool<T, NT, REP, I, 1>), dim3(grid), dim3(block), 0, L.stream, a, q);
+  else
+    hipLaunchKernelGGL((k_tr_eval_pool<T, NT, REP, I, 0>), dim3(grid), dim3(block), 0, L.stream, a, q);
+}
+template <typename T, int NT, int REP, int I>
+static void tr_pair_launch(const Launch &L, const TrArgs<T> &a, const TrArgs<T> &a2, int block) {
+  const int grid = grid_for(k_tr_eval2<T, NT, REP, I, 0>, block, 2 * a.N, L.num_cu);
+  if (L.profiled)
+    hipLaunchKernelGGL((k_tr_eval2<T, NT, REP, I, 1>), dim3(grid), dim3(block), 0, L.stream, a, a2);
+  else
+    hipLaunchKernelGGL((k_tr_eval2<T, NT, REP, I, 0>), dim3(grid), dim3(block), 0, L.stream, a, a2);
+}
+// Few waves on a CU, with the default table: workgroups of at most 256 threads, or
+// 512 threads twice on a CU at most (RELUs of 512 elements per CU 84.5 against 85.4
+// us, TRSLACKs 33.6 against 34.2).  384 threads (129 to 192 elements per CU) stay
+// in phases, where long Z_2^64 gates lose 5% otherwise (100 against 105 us), and
+// so do 512 beside other streams' launches (Z_2^64, B = 16 in 3 lanes: 1% slower).
+static bool tr_few(const Launch &L, int block, size_t n) {
+  return block <= 256 || (block == 512 && !L.shared && n <= size_t(block) * size_t(L.num_cu));
+}
+
 // One gate evaluation of both parties with prepared arguments: the regular
 // kernels, or (q set) their max-pool form.
 template <typename T>
@@ -1080,15 +1124,20 @@ static hipError_t tr_eval_launch(const Launch &L, const TrArgs<T> &a, const TrPo
     const int block = tr_eval_block(L, a.N);
     // a workgroup holds both parties' threads for block/2 elements
     if (block < 128 || block > 2 * kTrMaxTile || block % 128 != 0) return hipErrorInvalidConfiguration;
-    const int grid = grid_for(k_tr_eval<T, NT, REP, 0>, block, 2 * a.N, L.num_cu);
-    if (q && L.profiled)
-      hipLaunchKernelGGL((k_tr_eval_pool<T, NT, REP, 1>), dim3(grid), dim3(block), 0, L.stream, a, *q);
-    else if (q)
-      hipLaunchKernelGGL((k_tr_eval_pool<T, NT, REP, 0>), dim3(grid), dim3(block), 0, L.stream, a, *q);
-    else if (L.profiled)
-      hipLaunchKernelGGL((k_tr_eval<T, NT, REP, 1>), dim3(grid), dim3(block), 0, L.stream, a);
+    if constexpr (NT == 2 && REP == 32)
+      if (tr_few(L, block, a.N)) {
+        if (q)
+          tr_pool_launch<T, NT, REP, kFew>(L, a, *q, block);
+        else
+          tr_one_launch<T, NT, REP, kFew>(L, a, block);
+        return hipGetLastError();
+      }
+    if (q)
+      tr_pool_launch<T, NT, REP, kMid>(L, a, *q, block);
+    else if (block > 512)
+      tr_one_launch<T, NT, REP, kWide>(L, a, block);
     else
-      hipLaunchKernelGGL((k_tr_eval<T, NT, REP, 0>), dim3(grid), dim3(block), 0, L.stream, a);
+      tr_one_launch<T, NT, REP, kMid>(L, a, block);
     return hipGetLastError();
   });
 }
@@ -1210,11 +1259,12 @@ hipError_t launch_tr_eval2(const Launch &L, const TrLayout &lay, const TrLayout 
     }
     const int block = tr_eval_block(L, lay.N);
     if (block < 128 || block > 2 * kTrMaxTile || block % 128 != 0) return hipErrorInvalidConfiguration;
-    const int grid = grid_for(k_tr_eval2<T, NT, REP, 0>, block, 2 * lay.N, L.num_cu);
-    if (L.profiled)
-      hipLaunchKernelGGL((k_tr_eval2<T, NT, REP, 1>), dim3(grid), dim3(block), 0, L.stream, a, a2);
-    else
-      hipLaunchKernelGGL((k_tr_eval2<T, NT, REP, 0>), dim3(grid), dim3(block), 0, L.stream, a, a2);
+    if constexpr (NT == 2 && REP == 32)
+      if (tr_few(L, block, lay.N)) {
+        tr_pair_launch<T, NT, REP, kFew>(L, a, a2, block);
+        return hipGetLastError();
+      }
+    tr_pair_launch<T, NT, REP, kMid>(L, a, a2, block);
     return hipGetLastError();
   });
 }

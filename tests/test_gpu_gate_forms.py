@@ -53,6 +53,39 @@ def test_gate_form_edges(mp, num_cu, bw, kind, per_cu, extra):
         c.close()
 
 
+@pytest.mark.parametrize("per_cu,extra", [(65, 0), (128, 0), (128, 1), (192, 0), (192, 1), (256, 1), (512, 0), (512, 1)])
+@pytest.mark.parametrize("bw,kind", [(32, "RELU"), (32, "TRSLACK"), (64, "EXT"), (64, "RELU")])
+def test_one_lane_instance_edges(mp, num_cu, bw, kind, per_cu, extra):
+    """The one-lane kernel's workgroups of 256, 384 and 512 threads, and past 512
+    elements per CU the instance with its reads in phases."""
+    n = per_cu * num_cu + extra
+    c = mp.Ctx(bw=bw, scale=S)
+    try:
+        code = getattr(mp, kind)
+        assert c.tr_eval_form(code, n) == 0
+        x, r, xhat = _inputs(n, bw, 1 << (bw - S - 1 if kind == "EXT" else bw - 2), n + code)
+        k0, k1, ro = c.tr_keygen(code, r, seed=15, gate=2)
+        got = _signed((c.tr_eval(code, k0, k1, xhat).astype(np.uint64) - ro.astype(np.uint64)), bw)
+        assert np.array_equal(got, np.maximum(x, 0) if kind == "RELU" else x >> S if kind == "TRSLACK" else x)
+    finally:
+        c.close()
+
+
+@pytest.mark.parametrize("bw", [32, 64])
+@pytest.mark.parametrize("per_cu,extra", [(128, 0), (128, 1), (256, -1), (512, 0), (512, 1)])
+def test_maxpool_instance_edges(mp, num_cu, bw, per_cu, extra):
+    """One level of pairs at the same lines."""
+    C = per_cu * num_cu + extra
+    c = mp.Ctx(bw=bw, scale=S)
+    try:
+        x, r, xhat = _inputs(2 * C, bw, 1 << (bw - 3), C)
+        k0, k1, ro = c.maxpool_keygen(1, 2, C, r, seed=6, gate=2)
+        got = _signed(c.maxpool_eval(1, 2, C, k0, k1, xhat).astype(np.uint64) - ro.astype(np.uint64), bw)
+        assert np.array_equal(got, x.reshape(2, C).max(0))
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("extra", [-1, 65])
 def test_maxpool_form_edges(mp, num_cu, extra):
     """One level of pairs at the eight-wave line, the odd last row carried."""
