@@ -613,8 +613,12 @@ __global__ void __launch_bounds__(1024, W) k_tr_eval_b(TrArgs<T> a) {
   if (a.prio) __builtin_amdgcn_s_setprio(2);
   tr_eval_both<T, NT, REP, false, false>(a, a, TrPool<T>{});
 }
-template <typename T, int NT, int REP, int W, int TAG>
-__global__ void __launch_bounds__(1024, W) k_tr_eval2_b(TrArgs<T> a, TrArgs<T> a2) {
+// Pairs run in this form in lanes of at most 8 samples, whose other kernels share
+// the CU: 96 registers (16 spilled) leave them wave slots that 114 do not (B = 24 in
+// 3 lanes 2.44 -> 2.33 ms, 16 1.74 -> 1.69, 9 in 2 1.22 -> 1.18; 80 registers lose
+// 4% at 9 in 2 lanes).
+template <typename T, int NT, int REP, int TAG>
+__global__ void __launch_bounds__(1024, 5) k_tr_eval2_b(TrArgs<T> a, TrArgs<T> a2) {
   if (a.prio) __builtin_amdgcn_s_setprio(2);
   tr_eval_both<T, NT, REP, true, false>(a, a2, TrPool<T>{});
 }
@@ -1113,7 +1117,10 @@ static hipError_t tr_eval_launch(const Launch &L, const TrArgs<T> &a, const TrPo
   return with_variant(L, [&](auto v) {
     constexpr int NT = decltype(v)::nt, REP = decltype(v)::rep;
     if constexpr (sizeof(T) == 4) {
-      if (tr_form(L, a) == kFormBoth) {
+      // a max-pool level beside other lanes stays in one-lane workgroups, which leave
+      // those lanes room: the lanes with a level this large have 7 or 8 samples, and
+      // B = 20 in 3 of them takes 2.02 against 2.09 ms
+      if (tr_form(L, a) == kFormBoth && !(q && L.shared)) {
         if (both_waves(L, a) == 8)
           tr_both_launch<T, NT, REP, 8>(L, a, q);
         else
@@ -1249,11 +1256,11 @@ hipError_t launch_tr_eval2(const Launch &L, const TrLayout &lay, const TrLayout 
     if constexpr (sizeof(T) == 4) {
       const int bb = both_block(L, a) ? both_block(L, a2) : 0;
       if (bb) {
-        const int grid = grid_for(k_tr_eval2_b<T, NT, REP, 4, 0>, bb, lay.N, L.num_cu);
+        const int grid = grid_for(k_tr_eval2_b<T, NT, REP, 0>, bb, lay.N, L.num_cu);
         if (L.profiled)
-          hipLaunchKernelGGL((k_tr_eval2_b<T, NT, REP, 4, 1>), dim3(grid), dim3(bb), 0, L.stream, a, a2);
+          hipLaunchKernelGGL((k_tr_eval2_b<T, NT, REP, 1>), dim3(grid), dim3(bb), 0, L.stream, a, a2);
         else
-          hipLaunchKernelGGL((k_tr_eval2_b<T, NT, REP, 4, 0>), dim3(grid), dim3(bb), 0, L.stream, a, a2);
+          hipLaunchKernelGGL((k_tr_eval2_b<T, NT, REP, 0>), dim3(grid), dim3(bb), 0, L.stream, a, a2);
         return hipGetLastError();
       }
     }
