@@ -515,20 +515,35 @@ struct Runner {
 // ---------------------------------------------------------------------------
 // dealer: keys of gates at a cursor, written into resident arenas
 // ---------------------------------------------------------------------------
-// Device memory of a dealer run, kept between runs: take() hands out ranges in
-// order, and a run of the same sizes gets the ranges of the one before.
+// Device memory of a dealer run, handed out in order by take() and kept between
+// runs: a run of the same sizes gets the ranges of the one before, one of a smaller
+// batch fits the same chunks (every request is at most the larger run's, so it never
+// falls behind it), and a larger batch starts over, so that the chunks are never
+// more than one run's.  end() gives back what is more than kKeep.
 template <typename T>
 struct MaskPool {
+  static constexpr size_t kKeep = size_t(256) << 20;  // bytes per lane: a batch of some 85 samples in Z_2^32
   struct Chunk {
     DevBuf<T> buf;
     size_t n = 0;
   };
   std::vector<std::unique_ptr<Chunk>> chunks;
   size_t cur = 0, off = 0;
-  void reset() { cur = off = 0; }
+  int B = 0;  // the largest batch since the chunks were empty
+  void begin(int B_) {
+    if (B_ > B) release();
+    B = std::max(B, B_);
+    cur = off = 0;
+  }
+  void end() {
+    size_t n = 0;
+    for (auto &c : chunks) n += c->n;
+    if (n * sizeof(T) > kKeep) release();
+  }
   void release() {
     chunks.clear();
-    reset();
+    cur = off = 0;
+    B = 0;
   }
   hipError_t take(size_t n, T **p) {
     constexpr size_t kUnit = 256 / sizeof(T), kChunk = (size_t(16) << 20) / sizeof(T);
@@ -1022,11 +1037,11 @@ class Model final : public ModelBase, KeySource {
     have_pk_ = false;
     TRY(hipStreamSynchronize(L_.stream));  // a running forward may still read the arena
     drop_graph();
+    gen_.begin(B);
     TRY(ensure_arena(B));
     TRY(ensure_work(B));
     const int N = d_.n_nodes;
     const size_t BN = size_t(B) * N, BNN = BN * N;
-    gen_.reset();
     auto take = [&](size_t n, T **p) { return gen_.take(n, p); };
     // every gate's output mask first: PRF blocks that depend on nothing
     GenBatch<T> batch;
@@ -1124,6 +1139,7 @@ class Model final : public ModelBase, KeySource {
   }
   hipError_t keygen_end(int B, uint64_t seed) override {
     TRY(hipStreamSynchronize(L_.stream));
+    gen_.end();
     for (int p = 0; p < 2; p++) party_key_bytes(L_, seed, p, pk_[p]);
     have_pk_ = true;
     keyed_B_ = B;
@@ -1137,6 +1153,7 @@ class Model final : public ModelBase, KeySource {
     TRY(hipStreamSynchronize(L_.stream));  // a running forward may still read the arena
     keyed_B_ = -1;  // until the new keys are complete
     drop_graph();
+    gen_.release();
     TRY(ensure_arena(B));
     TRY(hipMemcpy(arena_[0], k0, bytes, hipMemcpyHostToDevice));
     TRY(hipMemcpy(arena_[1], k1, bytes, hipMemcpyHostToDevice));
@@ -1248,6 +1265,7 @@ class Model final : public ModelBase, KeySource {
     if (cs_) TRY(hipStreamSynchronize(cs_));
     free_stream();
     free_arena();  // the two slots replace the resident arena
+    gen_.release();
     gates_ = plan(B);
     // chunks: maximal runs of consecutive gates that fit in one slot
     chunks_.clear();
@@ -1570,6 +1588,7 @@ class Model final : public ModelBase, KeySource {
     TRY(hipStreamSynchronize(L_.stream));
     drop_graph();
     free_arena();
+    gen_.release();
     keyed_B_ = input_B_ = -1;
     have_pk_ = false;
     party_ = party;

@@ -1,0 +1,72 @@
+"""Device memory around a dealer's run: what a model keeps of it afterwards, and
+what it gives back when its keys come from elsewhere.  Sizes are differences of the
+device's used memory, which the allocator rounds to a few MiB."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+MIB = 1 << 20
+
+
+def _used():
+    import torch
+    torch.cuda.synchronize()
+    free, total = torch.cuda.mem_get_info()
+    return total - free
+
+
+def _model(mpcx, synth, B, bw):
+    wl = synth.workload(B, synth.Dims(bw=bw), seed=4)
+    c = mpcx.Ctx(bw=bw, scale=12)
+    return c, wl, lambda lanes=1: mpcx.Model(c, wl.dims, wl.W, lanes=lanes)
+
+
+def _forward(m, wl, B):
+    m.set_inputs(B, *wl.shares["x"], *wl.shares["a"], *wl.shares["m"], wl.prot)
+    m.forward(B)
+    return m.output(B)
+
+
+@pytest.mark.parametrize("how", ["stream", "import"])
+def test_other_keys_give_the_dealing_memory_back(synth, how):
+    """A model that dealt, then took its keys from host buffers, holds what one
+    holds that never dealt (the masks of a run of 8 samples are 23 MiB)."""
+    import mpcx
+    B = 8
+    c, wl, make = _model(mpcx, synth, B, 32)
+    d = make()
+    d.keygen(B, 5)
+    k0, k1 = d.export_keys(0, B), d.export_keys(1, B)
+    want = _forward(d, wl, B)
+    d.close()
+    held = []
+    for dealt in (False, True):
+        before = _used()
+        m = make()
+        if dealt:
+            m.keygen(B, 6)
+        if how == "stream":
+            m.attach_host_keys(B, k0, k1, 256 * MIB)
+        else:
+            m.import_keys(B, k0, k1)
+        assert np.array_equal(_forward(m, wl, B), want)
+        held.append(_used() - before)
+        m.close()
+    assert held[1] - held[0] <= 8 * MIB
+    c.close()
+
+
+def test_dealing_memory_kept_is_bounded(synth):
+    """Past 256 MiB of masks (50 samples in Z_2^64) a lane keeps none of them,
+    however many runs it has had."""
+    import mpcx
+    c, wl, make = _model(mpcx, synth, 1, 64)
+    m = make()
+    for B in (50, 60, 70):
+        m.keygen(B, B)
+        u = _used()
+    arena = 2 * m.key_bytes(70)
+    m.release_arena()
+    assert u - _used() <= arena + 256 * MIB + 16 * MIB
+    m.close()
+    c.close()
