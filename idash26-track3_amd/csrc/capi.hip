@@ -554,12 +554,15 @@ static mpcx_status maxpool_keygen_t(mpcx_ctx *c, int B, int N, int C, const void
   TrLayout lay[kMaxPoolLevels];
   int pairs[kMaxPoolLevels];
   const int Lv = maxpool_plan(c, B, N, C, lay, pairs);
-  const size_t rows = size_t(B) * N * C;
+  // the running masks' two planes: the first and second level's rows, which later
+  // levels' fit into in turn
+  const int r1 = N / 2 + (N & 1), r2 = r1 / 2 + (r1 & 1);
+  const size_t n1 = size_t(B) * r1 * C, n2 = size_t(B) * r2 * C;
   size_t np = 0;  // pairs of all levels
   for (int l = 0; l < Lv; l++) np += lay[l].N;
   void *sp = nullptr;
-  HIPC(c, ctx_work(c, (2 * rows + 2 * np) * sizeof(T), &sp), "hipMalloc");
-  T *va = static_cast<T *>(sp), *vb = va + rows, *dm = vb + rows, *ym = dm + np;
+  HIPC(c, ctx_work(c, (n1 + n2 + 2 * np) * sizeof(T), &sp), "hipMalloc");
+  T *va = static_cast<T *>(sp), *vb = va + n1, *dm = vb + n2, *ym = dm + np;
   const T *cur = static_cast<const T *>(in_mask);
   T *nxt = va;
   // every level's output masks are PRF blocks and come first; the levels' input

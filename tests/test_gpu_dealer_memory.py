@@ -70,3 +70,24 @@ def test_dealing_memory_kept_is_bounded(synth):
     assert u - _used() <= arena + 256 * MIB + 16 * MIB
     m.close()
     c.close()
+
+
+@pytest.mark.parametrize("bw,B,N,C", [(64, 64, 140, 312), (32, 256, 7, 1024), (64, 4096, 5, 128)])
+def test_maxpool_dealing_workspace(bw, B, N, C):
+    """At most three times the input's size (all levels' pairs twice, and the two
+    planes of running masks)."""
+    import mpcx
+    import torch
+    c = mpcx.Ctx(bw=bw, scale=12)
+    t = torch.int32 if bw == 32 else torch.int64
+    r = torch.arange(B * N * C, device="cuda").to(t)
+    ro = torch.zeros(B * C, dtype=t, device="cuda")
+    kb = c.lib.mpcx_maxpool_key_bytes(c.h, B, N, C)
+    k0, k1 = mpcx.empty_dev(kb), mpcx.empty_dev(kb)
+    p = mpcx.dptr
+    # the first level's keys alone: the kernel's own memory (spilled registers) is there
+    c.check(c.lib.mpcx_tr_keygen(c.h, mpcx.RELU, B * (N // 2) * C, p(r), p(r), 3, 1, p(k0), p(k1)), "tr_keygen")
+    before = _used()
+    c.check(c.lib.mpcx_maxpool_keygen(c.h, B, N, C, p(r), p(ro), 3, 1, p(k0), p(k1)), "maxpool_keygen")
+    assert _used() - before <= 3 * r.numel() * (bw // 8) + 4 * MIB
+    c.close()
