@@ -59,6 +59,10 @@ struct Launch {
   // model forwards with resident keys are captured once per batch size into a
   // HIP graph and replayed (0 = enqueue every kernel each time)
   int graph = 1;
+  // most bytes of masks that a model's lane holds at once while it deals
+  // (MPCX_DEAL_MIB); a key set that needs more, or more than the device has, is
+  // dealt gate by gate
+  size_t deal_bytes = SIZE_MAX;
   // the dealer's 16-byte key (dealer_key): set, or the seed alone
   bool has_dealer_key = false;
   uint8_t dealer_key[16] = {};

@@ -95,9 +95,11 @@ class ModelBase {
  public:
   virtual ~ModelBase() = default;
   virtual size_t key_bytes(int B) const = 0;
-  // a dealer run, enqueued on the lane's stream, and its completion
-  virtual hipError_t keygen_begin(int B, uint64_t seed) = 0;
+  // a dealer run, enqueued on the lane's stream (tight: in the least memory), and its
+  // completion; release_masks() gives back the memory that runs keep
+  virtual hipError_t keygen_begin(int B, uint64_t seed, bool tight) = 0;
   virtual hipError_t keygen_end(int B, uint64_t seed) = 0;
+  virtual void release_masks() = 0;
   virtual hipError_t import_keys(int B, const void *k0, const void *k1, size_t bytes) = 0;
   virtual hipError_t export_keys(int party, void *dst, size_t bytes) = 0;
   virtual hipError_t release_arena() = 0;

@@ -528,25 +528,43 @@ struct MaskPool {
     size_t n = 0;
   };
   std::vector<std::unique_ptr<Chunk>> chunks;
-  size_t cur = 0, off = 0;
+  size_t cur = 0, off = 0, held = 0;
   int B = 0;  // the largest batch since the chunks were empty
-  void begin(int B_) {
-    if (B_ > B) release();
+  // A tight run, for a device that a whole run's masks do not fit: every range is an
+  // allocation of its own, freed by drop() once nothing reads it any more (a chunk's
+  // ranges stay until the next run).
+  bool tight = false;
+  std::vector<std::unique_ptr<DevBuf<T>>> own;
+  size_t limit = SIZE_MAX;  // bytes of chunks
+  void begin(int B_, bool tight_) {
+    if (B_ > B || tight_) release();
+    tight = tight_;
     B = std::max(B, B_);
     cur = off = 0;
   }
   void end() {
-    size_t n = 0;
-    for (auto &c : chunks) n += c->n;
-    if (n * sizeof(T) > kKeep) release();
+    if (tight || held * sizeof(T) > kKeep) release();
   }
   void release() {
     chunks.clear();
-    cur = off = 0;
+    own.clear();
+    cur = off = held = 0;
     B = 0;
+  }
+  hipError_t drop(hipStream_t st, const T *p) {
+    if (!tight) return hipSuccess;
+    TRY(hipStreamSynchronize(st));
+    own.erase(std::remove_if(own.begin(), own.end(), [p](const auto &b) { return b->p == p; }), own.end());
+    return hipSuccess;
   }
   hipError_t take(size_t n, T **p) {
     constexpr size_t kUnit = 256 / sizeof(T), kChunk = (size_t(16) << 20) / sizeof(T);
+    if (tight) {
+      own.push_back(std::make_unique<DevBuf<T>>());
+      TRY(own.back()->alloc(n));
+      *p = own.back()->p;
+      return hipSuccess;
+    }
     n = (n + kUnit - 1) / kUnit * kUnit;
     while (cur < chunks.size() && off + n > chunks[cur]->n) {
       cur++;
@@ -555,8 +573,10 @@ struct MaskPool {
     if (cur == chunks.size()) {
       auto c = std::make_unique<Chunk>();
       const size_t want = std::max(n, kChunk);
+      if ((held + want) * sizeof(T) > limit) return hipErrorOutOfMemory;
       TRY(c->buf.alloc(want));
       c->n = want;
+      held += want;
       chunks.push_back(std::move(c));
     }
     *p = chunks[cur]->buf.p + off;
@@ -583,6 +603,7 @@ struct Dealer {
   uint8_t *K0, *K1;
   Cursor c;
   GenBatch<T> *batch = nullptr;
+  MaskPool<T> *pool = nullptr;
 
   hipError_t reveal(size_t n, T *mask) {
     RevealLayout lay = reveal_layout(bw, n, c.off);
@@ -591,7 +612,8 @@ struct Dealer {
     c.gate++;
     return hipSuccess;
   }
-  // own: the output mask's place without a batch; *out: where it is
+  // own: the output mask's place without a batch (null: taken from the pool);
+  // *out: where it is
   hipError_t tr(int kind, size_t n, const T *in, T *own, const T **out) {
     TrLayout lay = tr_layout(kind, bw, s, n, c.off);
     if (batch) {
@@ -601,6 +623,7 @@ struct Dealer {
       it.in = in;
       *out = it.out;
     } else {
+      if (!own) TRY(pool->take(n, &own));
       TRY(launch_tr_keygen<T>(L, lay, seed, c.gate, in, own, K0, K1));
       *out = own;
     }
@@ -816,13 +839,16 @@ class Model final : public ModelBase, KeySource {
     if (!local_trunc()) {
       const T *y = nullptr;
       TRY(d.tr(G_TRMOD, n, rin, nullptr, &y));
-      return d.tr(relu ? G_EXTRELU : G_EXT, n, y, nullptr, rout);
+      TRY(d.tr(relu ? G_EXTRELU : G_EXT, n, y, nullptr, rout));
+      return gen_.drop(L_.stream, y);
     }
     T *y = nullptr;
     TRY(gen_.take(n, &y));
     TRY(launch_local_ars<T>(L_, n, s_, rin, nullptr, 1, y));
     *rout = y;
-    return relu ? d.tr(G_RELU, n, y, nullptr, rout) : hipSuccess;
+    if (!relu) return hipSuccess;
+    TRY(d.tr(G_RELU, n, y, nullptr, rout));
+    return gen_.drop(L_.stream, y);
   }
 
   // ---------------- weights ----------------
@@ -1029,24 +1055,27 @@ class Model final : public ModelBase, KeySource {
     return hipSuccess;
   }
 
-  // Enqueues a dealer run on the lane's stream; keygen_end waits for it.
-  hipError_t keygen_begin(int B, uint64_t seed) override {
+  // Enqueues a dealer run on the lane's stream; keygen_end waits for it.  tight:
+  // gate by gate, holding no mask longer than it is read (MaskPool).
+  hipError_t keygen_begin(int B, uint64_t seed, bool tight) override {
     if (party_ >= 0) return hipErrorNotSupported;  // the dealer holds both parties' keys
     TRY(leave_stream());
     keyed_B_ = -1;  // until the new keys are complete
     have_pk_ = false;
     TRY(hipStreamSynchronize(L_.stream));  // a running forward may still read the arena
     drop_graph();
-    gen_.begin(B);
+    gen_.limit = L_.deal_bytes;
+    gen_.begin(B, tight);
     TRY(ensure_arena(B));
     TRY(ensure_work(B));
     const int N = d_.n_nodes;
     const size_t BN = size_t(B) * N, BNN = BN * N;
     auto take = [&](size_t n, T **p) { return gen_.take(n, p); };
+    auto drop = [&](const T *p) { return gen_.drop(L_.stream, p); };
     // every gate's output mask first: PRF blocks that depend on nothing
     GenBatch<T> batch;
     for (const GateKey &g : plan(B)) {
-      if (!g.tr_kind) continue;
+      if (!g.tr_kind || tight) continue;
       TrGenItem<T> it;
       it.lay = tr_layout(g.tr_kind, bw_, s_, g.n, g.begin);
       it.gate = g.gate;
@@ -1054,7 +1083,7 @@ class Model final : public ModelBase, KeySource {
       batch.items.push_back(it);
     }
     TRY(launch_tr_masks<T>(L_, seed, batch.items.data(), batch.items.size()));
-    Dealer<T> d{L_, bw_, s_, seed, arena_[0], arena_[1], Cursor{}, &batch};
+    Dealer<T> d{L_, bw_, s_, seed, arena_[0], arena_[1], Cursor{}, tight ? nullptr : &batch, &gen_};
     auto pub_gemm = [&](const T *x, int l, size_t rows, T **y) -> hipError_t {
       int in, out;
       layer_io(l, &in, &out);
@@ -1078,31 +1107,40 @@ class Model final : public ModelBase, KeySource {
     TRY(d.reveal(BN * d_.feat, rX));
     TRY(d.reveal(BN, rm));
     TRY(adj_.keygen(d, rA, rN));
+    TRY(drop(rA));
     // GCN stack; x is the running activation mask
     const T *x = rX, *y = nullptr;
     for (int l = 0; l < 3; l++) {
       const int fo = d_.gcn[l];
       const size_t En = BN * fo;
       TRY(pub_gemm(x, l, BN, &z));
+      TRY(drop(x));
       if (xw_slack())
         TRY(d.tr(G_TRSLACK, En, z, nullptr, &y));
       else
         TRY(trunc_keygen(d, false, En, z, &y));
+      TRY(drop(z));
       TRY(take(En, &z));
       TRY(d.sxs(B, N, N, fo, rN, y, z, tmp));
+      TRY(drop(y));
       if (agg_split()) {
         TRY(d.tr(G_TRSLACK, En, z, nullptr, &y));
         TRY(d.tr(G_RELUSLACK, En, y, nullptr, &x));
+        TRY(drop(y));
       } else {
         TRY(trunc_keygen(d, true, En, z, &x));
       }
+      TRY(drop(z));
     }
+    TRY(drop(rN));
+    TRY(drop(tmp));
     // pool
     const int C = d_.gcn[2];
     const T Sm = T(1) << (pool_sentinel_bit() - d_.mask_scale);
     T *cur, *dm, *nxt;
     TRY(take(BN * C, &cur));
     TRY(launch_pool_prep<T>(L_, BN, C, x, rm, Sm, T(0), cur));
+    TRY(drop(x));
     int pairs[32];
     const int Lv = pool_levels(N, pairs);
     int R = N;
@@ -1111,8 +1149,15 @@ class Model final : public ModelBase, KeySource {
       const size_t En = size_t(B) * pr * C;
       TRY(take(En, &dm));
       TRY(take(size_t(B) * (pr + (R & 1)) * C, &nxt));
-      TRY(d.tr(pool_kind(), En, dm, nullptr, &y));
-      TRY(launch_pool_masks<T>(L_, B, R, C, cur, y, dm, nxt));
+      if (tight) {  // the gate's keys need its input mask now
+        TRY(launch_pool_diff<T>(L_, B, R, C, cur, dm));
+        TRY(d.tr(pool_kind(), En, dm, nullptr, &y));
+        TRY(launch_pool_combine<T>(L_, B, R, C, cur, y, nullptr, nxt));
+      } else {
+        TRY(d.tr(pool_kind(), En, dm, nullptr, &y));
+        TRY(launch_pool_masks<T>(L_, B, R, C, cur, y, dm, nxt));
+      }
+      for (const T *done : {static_cast<const T *>(dm), y, static_cast<const T *>(cur)}) TRY(drop(done));
       cur = nxt;
       R = pr + (R & 1);
     }
@@ -1136,6 +1181,10 @@ class Model final : public ModelBase, KeySource {
     if (d.c.off != key_bytes(B) || d.c.gate != uint32_t(plan(B).size()) + 1 || batch.next != batch.items.size())
       return hipErrorUnknown;
     return launch_tr_keygen_batch<T>(L_, seed, batch.items.data(), batch.items.size(), arena_[0], arena_[1]);
+  }
+  void release_masks() override {
+    (void)hipStreamSynchronize(L_.stream);
+    gen_.release();
   }
   hipError_t keygen_end(int B, uint64_t seed) override {
     TRY(hipStreamSynchronize(L_.stream));
@@ -2058,12 +2107,24 @@ size_t LaneSet::unique_key_bytes(int B, int party) const {
 hipError_t LaneSet::keygen(int B, uint64_t seed) {
   keyed_B_ = -1;
   // the lanes' runs side by side, then waited for; a failed run leaves none behind
-  hipError_t e = each(B, [&](int i, int Bi, int) { return lane_[i]->keygen_begin(Bi, lane_seed(seed, i)); });
-  if (e != hipSuccess) {
+  hipError_t e = each(B, [&](int i, int Bi, int) { return lane_[i]->keygen_begin(Bi, lane_seed(seed, i), false); });
+  if (e != hipSuccess)
     for (size_t i = 0; i < st_.size(); i++) (void)hipStreamSynchronize(st_[i]);
+  if (e == hipErrorOutOfMemory) {
+    // the masks of all gates and lanes at once do not fit: lane by lane, gate by gate
+    (void)hipGetLastError();
+    for (auto *m : lane_) m->release_masks();
+    e = each(B, [&](int i, int Bi, int) {
+      TRY(lane_[i]->keygen_begin(Bi, lane_seed(seed, i), true));
+      return lane_[i]->keygen_end(Bi, lane_seed(seed, i));
+    });
+  } else if (e == hipSuccess) {
+    e = each(B, [&](int i, int Bi, int) { return lane_[i]->keygen_end(Bi, lane_seed(seed, i)); });
+  }
+  if (e != hipSuccess) {
+    for (auto *m : lane_) m->release_masks();
     return e;
   }
-  TRY(each(B, [&](int i, int Bi, int) { return lane_[i]->keygen_end(Bi, lane_seed(seed, i)); }));
   keyed_B_ = B;
   return hipSuccess;
 }

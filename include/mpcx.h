@@ -93,8 +93,10 @@ typedef struct mpcx_model mpcx_model;
  * wide-K matrix-core kernels where they apply, the tiled matrix-core kernels
  * elsewhere), wide (the same without the panel kernel), tiled (the tiled
  * matrix-core kernels only) or valu (the VALU kernels); MPCX_GRAPH = 0 (model
- * forwards enqueue every kernel instead of replaying a captured HIP graph).  All
- * paths give the same results bit for bit. */
+ * forwards enqueue every kernel instead of replaying a captured HIP graph);
+ * MPCX_DEAL_MIB (MiB of masks that a lane of mpcx_model_keygen holds at most, by
+ * default what a key set needs; beyond it, or beyond the device's memory, keys are
+ * dealt gate by gate).  All paths give the same results bit for bit. */
 mpcx_status mpcx_create(int bw, int scale, int device, mpcx_ctx **out);
 void mpcx_destroy(mpcx_ctx *ctx);
 const char *mpcx_last_error(const mpcx_ctx *ctx);

@@ -91,3 +91,24 @@ def test_maxpool_dealing_workspace(bw, B, N, C):
     c.check(c.lib.mpcx_maxpool_keygen(c.h, B, N, C, p(r), p(ro), 3, 1, p(k0), p(k1)), "maxpool_keygen")
     assert _used() - before <= 3 * r.numel() * (bw // 8) + 4 * MIB
     c.close()
+
+
+@pytest.mark.parametrize("bw,B,lanes,slack,mib", [(32, 2, 1, 0, 0), (32, 3, 2, 1, 0), (32, 2, 1, 2, 0), (32, 2, 1, 3, 0),
+                                                  (64, 3, 2, 0, 0), (32, 8, 1, 0, 16), (32, 9, 2, 0, 12)])
+def test_gate_by_gate_dealing_writes_the_same_keys(synth, monkeypatch, bw, B, lanes, slack, mib):
+    """A lane that may hold no masks at once (0), or fewer than its run needs
+    (16 MiB: refused after the first chunk), deals gate by gate."""
+    import mpcx
+    keys = []
+    for limit in (None, str(mib)):
+        if limit is not None:
+            monkeypatch.setenv("MPCX_DEAL_MIB", limit)
+        wl = synth.workload(B, synth.Dims(bw=bw, slack=slack), seed=4)
+        c = mpcx.Ctx(bw=bw, scale=12)
+        m = mpcx.Model(c, wl.dims, wl.W, lanes=lanes)
+        m.keygen(B, 21)
+        keys.append([m.export_keys(p, B) for p in (0, 1)])
+        m.close()
+        c.close()
+    for a, b in zip(*keys):
+        assert np.array_equal(a, b)
