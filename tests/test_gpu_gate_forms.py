@@ -88,7 +88,8 @@ def test_maxpool_instance_edges(mp, num_cu, bw, per_cu, extra):
 
 @pytest.mark.parametrize("extra", [-1, 65])
 def test_maxpool_form_edges(mp, num_cu, extra):
-    """One level of pairs at the eight-wave line, the odd last row carried."""
+    """A first level of pairs at the eight-wave line, its odd last row carried to a
+    second one."""
     B, N, C = 1, 3, 4096 * num_cu + extra
     c = mp.Ctx(bw=32, scale=S)
     try:
@@ -101,16 +102,17 @@ def test_maxpool_form_edges(mp, num_cu, extra):
 
 
 @pytest.mark.parametrize("bw,kind,extra", [(32, "EXTRELU", -1), (32, "EXTRELU", 65), (64, "TRMOD", 1),
-                                           (64, "TRRELU", -63), (32, "DRELU", 0)])
+                                           (64, "TRRELU", -63), (32, "DRELU", 0), (32, "EXTRELU", -64),
+                                           (64, "TRRELU", -65), (32, "TR", -127)])
 def test_keygen_form_edges(mp, orc, num_cu, bw, kind, extra):
     """The dealer at the line between its 256- and 1024-thread workgroups (512
-    elements per CU): both keys and the output mask as the oracle's dealer writes
-    them, byte for byte."""
+    elements per CU, in tiles of 64: the last one below is 64 less): both keys and
+    the output mask as the oracle's dealer writes them, byte for byte."""
     n = 512 * num_cu + extra
     c = mp.Ctx(bw=bw, scale=S)
     try:
         code = getattr(mp, kind)
-        rin = _inputs(n, bw, 1, 77 + extra)[1]
+        rin = _inputs(n, bw, 1, n)[1]
         k0, k1, ro = c.tr_keygen(code, rin, seed=11, gate=4)
         o0, o1, oro = orc.tr_keygen(11, 4, code, bw, S, rin)
         assert np.array_equal(ro.astype(np.uint64), oro.astype(np.uint64))

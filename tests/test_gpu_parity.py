@@ -453,13 +453,10 @@ def test_mul_keys_and_eval(ctx, orc):
 
 
 def test_mul_and_reveal_in_place(ctx, orc, mp):
-    """Through the C ABI, outputs that overlap an input (the product over its own
-    x^ buffer, the reveal over party 0's share) give the same values: the C-ABI
-    calls always take the message path (messages, then the reconstruction), so
-    no thread writes an output while others still gather inputs.  The model's
-    own choice between that path and the one-launch evaluation (by whether the
-    output overlaps an input) is covered by the model parity tests, whose
-    products and reveals write disjoint buffers."""
+    """Through the C ABI, outputs that overlap an input: the product over its own
+    x^ buffer, which other threads gather, takes the message path (messages, then
+    the reconstruction); the reveal over party 0's share, which only the writing
+    thread reads, is one launch."""
     bw = ctx.bw
     rng = np.random.default_rng(bw + 5)
     nx, ny, nz = 3000, 200, 2500
@@ -489,6 +486,60 @@ def test_mul_and_reveal_in_place(ctx, orc, mp):
     ctx.check(ctx.lib.mpcx_reveal_eval(ctx.h, n, mp.dptr(r0), mp.dptr(r1), mp.dptr(d0), mp.dptr(d1), mp.dptr(d0)),
               "reveal_eval")
     assert np.array_equal(signed(mp.from_dev(d0, ctx.T, n).astype(np.uint64) - rm, bw), v)
+
+
+@pytest.mark.parametrize("shift", [0, 1, 64])
+def test_lut_and_reveal_overlapping_outputs(ctx, orc, mp, shift):
+    """The lookup over its own x^ (one launch) and shifted into it, over the table
+    and over a key, and the reveal shifted into either share: as into a buffer
+    apart."""
+    bw = ctx.bw
+    rng = np.random.default_rng(shift)
+    w = ctx.ring(np.zeros(1)).itemsize
+    n = 200  # at most the table's entries
+    table = orc.invsqrt_table(S, 138)
+    x = rng.integers(0, 256, n).astype(np.uint64)
+    rin = rmask(rng, n, bw)
+    k0, k1, ro = ctx.lut8_keygen(rin, seed=4, gate=6)
+    xh = ctx.ring((x + rin) & M(bw))
+    want = ctx.lut8_eval(k0, k1, table, xh)
+    assert np.array_equal((want.astype(np.uint64) - ro) & M(bw), table[x.astype(np.int64)])
+    pad = np.zeros(64, ctx.T)
+
+    def at(t, off):
+        return mp.C.c_void_p(t.data_ptr() + off * w)
+
+    def out_of(t, off):
+        return mp.from_dev(t, np.uint8)[off * w:(off + n) * w].view(ctx.T)
+
+    for over in ("x", "table", "key"):
+        dx, dt = mp.to_dev(np.concatenate([xh, pad])), mp.to_dev(np.concatenate([ctx.ring(table), pad]))
+        c0 = k0.clone()
+        mp._torch().cuda.synchronize()
+        t = {"x": dx, "table": dt, "key": c0}[over]
+        ctx.check(ctx.lib.mpcx_lut8_eval(ctx.h, n, mp.dptr(c0), mp.dptr(k1), mp.dptr(dt), mp.dptr(dx), at(t, shift)),
+                  "lut8_eval")
+        assert np.array_equal(out_of(t, shift), want), over
+    r0, r1, rm = ctx.reveal_keygen(n, seed=4, gate=7)
+    v0 = rmask(rng, n, bw)
+    v1 = (x - v0) & M(bw)
+    want = (x + rm.astype(np.uint64)) & M(bw)
+    for over in (0, 1):
+        d = [mp.to_dev(np.concatenate([ctx.ring(v), pad])) for v in (v0, v1)]
+        ctx.check(ctx.lib.mpcx_reveal_eval(ctx.h, n, mp.dptr(r0), mp.dptr(r1), mp.dptr(d[0]), mp.dptr(d[1]),
+                                           at(d[over], shift)), "reveal_eval")
+        assert np.array_equal(out_of(d[over], shift).astype(np.uint64), want), over
+
+
+@pytest.mark.parametrize("n", [1, 513, 300001])
+def test_lut8_and_reveal_keys_over_rounds(ctx, orc, n):
+    """One element, a ragged second workgroup, and several rounds of the grid."""
+    rin = rmask(np.random.default_rng(n), n, ctx.bw)
+    for got, want in ((ctx.lut8_keygen(rin, seed=14, gate=3), orc.lut8_keygen(14, 3, ctx.bw, rin)),
+                      (ctx.reveal_keygen(n, seed=15, gate=4), orc.reveal_keygen(15, 4, ctx.bw, n))):
+        for g, w in zip(got[:2], want[:2]):
+            assert np.array_equal(host(g)[:w.size], w)
+        assert np.array_equal(got[2].astype(np.uint64), np.asarray(want[2]).astype(np.uint64))
 
 
 def test_lut8_keys_and_eval(ctx, orc):
@@ -1098,6 +1149,23 @@ def test_adjnorm_keys_and_eval(mp, orc, synth, bw):
     got1 = c.adjnorm_eval(1, N, 138, g0s, g1s, a0[:1], a1[:1])
     want1, _ = orc.adjnorm_eval(bw, S, 1, N, 138, o0s, o1s, a0[:1], a1[:1])
     assert np.array_equal(got1.astype(np.uint64), want1)
+    assert np.array_equal(c.adjnorm_eval(B, N, 138, g0, g1, a0, a1).astype(np.uint64), want)
+    c.close()
+
+
+@pytest.mark.parametrize("bw,rows", [(32, 16), (64, 8)])
+@pytest.mark.parametrize("less", [0, 1])
+def test_adjnorm_tile_heights(mp, orc, synth, bw, rows, less):
+    """A (.) W on tiles of `rows` rows as soon as those are one per CU, and with one
+    graph less on tiles of two (N = 20: the last tile is ragged in both)."""
+    N = 20
+    B = -(-_num_cu() // -(-N // rows)) - less
+    _, A, _ = synth.molecules(B, synth.Dims(bw=bw, n_nodes=N), seed=8, min_atoms=3, max_atoms=N)
+    a0, a1 = synth.share(A, bw, 79)
+    c = mp.Ctx(bw=bw)
+    g0, g1, _ = c.adjnorm_keygen(B, N, seed=9)
+    o0, o1, _ = orc.adjnorm_keygen(bw, S, B, N, 9)
+    want, _ = orc.adjnorm_eval(bw, S, B, N, 138, o0, o1, a0, a1)
     assert np.array_equal(c.adjnorm_eval(B, N, 138, g0, g1, a0, a1).astype(np.uint64), want)
     c.close()
 
