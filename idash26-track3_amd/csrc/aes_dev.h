@@ -228,6 +228,61 @@ struct AesPerm {
     return o;
   }
 
+  // Two whitened blocks under one key: a round's 16 reads of one go out while the
+  // other's columns are formed, as in AesPerm2 (one after the other, which the
+  // scheduler makes of two calls, the dealer's gates take up to 1.7 times as long).
+  struct Reads {
+    uint32_t v[4][4];  // byte b of column j
+  };
+  __device__ __forceinline__ void read(Reads &r, uint4 c) const {
+    const uint32_t w[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      r.v[j][0] = L<0, 0>(w[j]);
+      r.v[j][1] = L<0, 1>(w[j]);
+      r.v[j][2] = L<0, 2>(w[j]);
+      r.v[j][3] = L<0, 3>(w[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ static uint32_t col(const Reads &r, int j, uint32_t k) {
+    return xor3(xor3(r.v[j][0], rot<1>(r.v[(j + 1) & 3][1]), rot<2>(r.v[(j + 2) & 3][2])),
+                rot<3>(r.v[(j + 3) & 3][3]), k);
+  }
+  __device__ __forceinline__ static uint4 cols(const Reads &r, const uint32_t *k) {
+    return make_uint4(col(r, 0, k[0]), col(r, 1, k[1]), col(r, 2, k[2]), col(r, 3, k[3]));
+  }
+  __device__ __forceinline__ static uint32_t last(const Reads &r, int j) {
+    const uint32_t lo = __builtin_amdgcn_perm(r.v[(j + 1) & 3][1], r.v[j][0], 0x0c0c0501u);
+    const uint32_t hi = __builtin_amdgcn_perm(r.v[(j + 3) & 3][3], r.v[(j + 2) & 3][2], 0x0c0c0501u);
+    return (hi << 16) | lo;
+  }
+  __device__ __forceinline__ static uint4 lasts(const Reads &r, const uint32_t *k) {
+    return make_uint4(last(r, 0) ^ k[0], last(r, 1) ^ k[1], last(r, 2) ^ k[2], last(r, 3) ^ k[3]);
+  }
+  __device__ __forceinline__ void rounds2(uint4 &u, uint4 &v, const AesRK &rk) const {
+    Reads a, b;
+    read(a, u);
+    read(b, v);
+#pragma unroll
+    for (int r = 1; r < 10; r++) {
+      read(a, cols(a, rk.w + 4 * r));
+      read(b, cols(b, rk.w + 4 * r));
+    }
+    u = lasts(a, rk.w + 40);
+    v = lasts(b, rk.w + 40);
+  }
+  __device__ __forceinline__ void enc2(uint4 u, uint4 v, const AesRK &rk, uint4 *eu, uint4 *ev) const {
+    *eu = make_uint4(u.x ^ rk.w[0], u.y ^ rk.w[1], u.z ^ rk.w[2], u.w ^ rk.w[3]);
+    *ev = make_uint4(v.x ^ rk.w[0], v.y ^ rk.w[1], v.z ^ rk.w[2], v.w ^ rk.w[3]);
+    rounds2(*eu, *ev, rk);
+  }
+  __device__ __forceinline__ void hash2(uint4 s, uint4 u, const AesRK &rk, uint4 *hs, uint4 *hu) const {
+    enc2(make_uint4(s.z, s.w, s.z ^ s.x, s.w ^ s.y), make_uint4(u.z, u.w, u.z ^ u.x, u.w ^ u.y), rk, hs, hu);
+    *hs = make_uint4(hs->x ^ s.z, hs->y ^ s.w, xor3(hs->z, s.z, s.x), xor3(hs->w, s.w, s.y));
+    *hu = make_uint4(hu->x ^ u.z, hu->y ^ u.w, xor3(hu->z, u.z, u.x), xor3(hu->w, u.w, u.y));
+  }
+
   // Dealer PRF block AES_kd(idx_lo, idx_hi, field, gate).
   __device__ __forceinline__ uint4 prf(const AesRK &kd, uint32_t gate, uint32_t field, uint64_t idx) const {
     uint4 b;
@@ -552,7 +607,7 @@ using AesLds = typename AesSel<NT, REP>::type;
 // Two dealer PRF blocks of one key, side by side where the table type can.
 template <class A>
 __device__ __forceinline__ void enc_pair(const A &aes, const AesRK &k, uint4 u, uint4 v, uint4 *eu, uint4 *ev) {
-  if constexpr (std::is_same<A, AesPerm2>::value) {
+  if constexpr (std::is_same<A, AesPerm2>::value || std::is_same<A, AesPerm>::value) {
     aes.enc2(u, v, k, eu, ev);
   } else {
     *eu = aes.enc(u, k);

@@ -828,13 +828,21 @@ static TrArgs<T> tr_args(const TrLayout &lay) {
   return a;
 }
 
-// One launch over ka.tiles tiles.  Few tiles go to 256-thread workgroups, whose
-// waves are spread over the CUs before a workgroup takes a second one.
+// Workgroup of a dealer launch over 64-element tiles.  As many as 256-thread
+// workgroups take in one round of the CUs (two a CU, one with the 128 KiB table, at
+// four tiles each) go to those, whose waves are spread over the CUs before a
+// workgroup takes a second one.
+template <int NT, int REP>
+static int gen_block(const Launch &L, size_t tiles) {
+  constexpr size_t kFit = 163840 / AesLds<NT, REP>::kBytes;
+  return L.aes_block > 0 ? L.aes_block : tiles < 4 * kFit * size_t(L.num_cu) ? 256 : 1024;
+}
+// One launch over ka.tiles tiles.
 template <typename T>
 static hipError_t tr_gen_launch(const Launch &L, const TrGenArgs<T> &ka) {
   return with_variant(L, [&](auto v) {
     constexpr int NT = decltype(v)::nt, REP = decltype(v)::rep;
-    const int block = L.aes_block > 0 ? L.aes_block : ka.tiles < 8 * size_t(L.num_cu) ? 256 : 1024;
+    const int block = gen_block<NT, REP>(L, ka.tiles);
     const int occ_grid = grid_for(k_tr_keygen<T, NT, REP>, block, size_t(-1) / 2, L.num_cu);
     const int grid = int(std::min<size_t>(size_t(occ_grid), ka.tiles));
     hipLaunchKernelGGL((k_tr_keygen<T, NT, REP>), dim3(grid), dim3(block), 0, L.stream, ka);
@@ -913,7 +921,7 @@ hipError_t launch_tr_masks(const Launch &L, uint64_t seed, const TrGenItem<T> *i
     if (a.tiles == 0) continue;
     const hipError_t e = with_variant(L, [&](auto v) {
       constexpr int NT = decltype(v)::nt, REP = decltype(v)::rep;
-      const int block = L.aes_block > 0 ? L.aes_block : a.tiles < 8 * size_t(L.num_cu) ? 256 : 1024;
+      const int block = gen_block<NT, REP>(L, a.tiles);
       const int occ_grid = grid_for(k_tr_masks<T, NT, REP>, block, size_t(-1) / 2, L.num_cu);
       const int grid = int(std::min<size_t>(size_t(occ_grid), a.tiles));
       hipLaunchKernelGGL((k_tr_masks<T, NT, REP>), dim3(grid), dim3(block), 0, L.stream, a);
