@@ -1149,7 +1149,7 @@ static hipError_t tr_eval_launch(const Launch &L, const TrArgs<T> &a, const TrPo
       }
     if (q)
       tr_pool_launch<T, NT, REP, kMid>(L, a, *q, block);
-    else if (block > 512)
+    else if (block > 512 && 2 * a.N > size_t(block) * size_t(L.num_cu))  // a second workgroup on a CU
       tr_one_launch<T, NT, REP, kWide>(L, a, block);
     else
       tr_one_launch<T, NT, REP, kMid>(L, a, block);
