@@ -442,39 +442,11 @@ struct AesPerm2 {
                       xor3(last(r, 2), rk.w[42], s.z) ^ s.x, xor3(last(r, 3), rk.w[43], s.w) ^ s.y);
   }
 
-  // One block in the scheduler's own order, which starts a column while the reads
-  // of the next ones are on their way: with a single chain a phase forms all four
-  // columns and then waits for all reads.  25 hashes one after another take 34
-  // against 41 us with one wave per SIMD, 42-45 in both orders with 1.5 and two and
-  // 72-73 with four; but the order needs more registers, and one held to 64 of them
-  // keeps few reads in flight (146 against 103 us for 64-bit ReLUs of 160 elements
-  // per CU).  So PRF blocks and the gates of small workgroups (AesPerm2Few) take
-  // this order, the other walks the phases.
-  __device__ __forceinline__ uint32_t col(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t k) const {
-    const uint32_t h = xor3(t0<2>(c), t1<3>(d), (k << 16) | (k >> 16));
-    return xor3(t0<0>(a), t1<1>(b), __builtin_amdgcn_alignbit(h, h, 16));
-  }
-  __device__ __forceinline__ uint32_t last(uint32_t a, uint32_t b, uint32_t c, uint32_t d) const {
-    const uint32_t lo = __builtin_amdgcn_perm(t0<1>(b), t0<0>(a), 0x0c0c0501u);
-    const uint32_t hi = __builtin_amdgcn_perm(t0<3>(d), t0<2>(c), 0x0c0c0501u);
-    return (hi << 16) | lo;
-  }
-  // the block from its whitened input to before the last round key
-  __device__ __forceinline__ uint4 block(uint4 c, const AesRK &rk) const {
-#pragma unroll
-    for (int r = 1; r < 10; r++) {
-      const uint32_t n0 = col(c.x, c.y, c.z, c.w, rk.w[4 * r + 0]);
-      const uint32_t n1 = col(c.y, c.z, c.w, c.x, rk.w[4 * r + 1]);
-      const uint32_t n2 = col(c.z, c.w, c.x, c.y, rk.w[4 * r + 2]);
-      const uint32_t n3 = col(c.w, c.x, c.y, c.z, rk.w[4 * r + 3]);
-      c = make_uint4(n0, n1, n2, n3);
-    }
-    return make_uint4(last(c.x, c.y, c.z, c.w), last(c.y, c.z, c.w, c.x), last(c.z, c.w, c.x, c.y),
-                      last(c.w, c.x, c.y, c.z));
-  }
   __device__ __forceinline__ uint4 enc(uint4 in, const AesRK &rk) const {
-    const uint4 o = block(whiten(in, rk), rk);
-    return make_uint4(o.x ^ rk.w[40], o.y ^ rk.w[41], o.z ^ rk.w[42], o.w ^ rk.w[43]);
+    Reads r;
+    start(r, whiten(in, rk));
+    rounds(r, rk);
+    return enc_out(r, rk);
   }
   __device__ __forceinline__ void enc2(uint4 u, uint4 v, const AesRK &rk, uint4 *eu, uint4 *ev) const {
     Reads a, b;
@@ -510,13 +482,50 @@ struct AesPerm2 {
   }
 };
 
-// AesPerm2 with single hashes in the scheduler's order (AesPerm2::block).
+// AesPerm2 with single blocks in the scheduler's own order, which starts a column
+// while the reads of the next ones are on their way: with a single chain a phase
+// forms all four columns and then waits for all reads.  25 hashes one after another
+// take 34 against 41 us with one wave per SIMD, 42-45 in both orders with 1.5 and two
+// and 72-73 with four; but the order needs more registers, and one held to 64 of them
+// keeps few reads in flight (146 against 103 us for 64-bit ReLUs of 160 elements per
+// CU).  For gates of few waves and for kernels that draw PRF blocks one by one; the
+// others, the gates' dealer among them (1.4 M EXTRELU keys 530 against 535 us), stay
+// in phases.
 struct AesPerm2Few : AesPerm2 {
   using AesPerm2::AesPerm2;
+  __device__ __forceinline__ uint32_t col(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t k) const {
+    const uint32_t h = xor3(t0<2>(c), t1<3>(d), (k << 16) | (k >> 16));
+    return xor3(t0<0>(a), t1<1>(b), __builtin_amdgcn_alignbit(h, h, 16));
+  }
+  __device__ __forceinline__ uint32_t last(uint32_t a, uint32_t b, uint32_t c, uint32_t d) const {
+    const uint32_t lo = __builtin_amdgcn_perm(t0<1>(b), t0<0>(a), 0x0c0c0501u);
+    const uint32_t hi = __builtin_amdgcn_perm(t0<3>(d), t0<2>(c), 0x0c0c0501u);
+    return (hi << 16) | lo;
+  }
+  // the block from its whitened input to before the last round key
+  __device__ __forceinline__ uint4 block(uint4 c, const AesRK &rk) const {
+#pragma unroll
+    for (int r = 1; r < 10; r++) {
+      const uint32_t n0 = col(c.x, c.y, c.z, c.w, rk.w[4 * r + 0]);
+      const uint32_t n1 = col(c.y, c.z, c.w, c.x, rk.w[4 * r + 1]);
+      const uint32_t n2 = col(c.z, c.w, c.x, c.y, rk.w[4 * r + 2]);
+      const uint32_t n3 = col(c.w, c.x, c.y, c.z, rk.w[4 * r + 3]);
+      c = make_uint4(n0, n1, n2, n3);
+    }
+    return make_uint4(last(c.x, c.y, c.z, c.w), last(c.y, c.z, c.w, c.x), last(c.z, c.w, c.x, c.y),
+                      last(c.w, c.x, c.y, c.z));
+  }
+  __device__ __forceinline__ uint4 enc(uint4 in, const AesRK &rk) const {
+    const uint4 o = block(whiten(in, rk), rk);
+    return make_uint4(o.x ^ rk.w[40], o.y ^ rk.w[41], o.z ^ rk.w[42], o.w ^ rk.w[43]);
+  }
   __device__ __forceinline__ uint4 hash(uint4 s, const AesRK &rk) const {
     const uint4 o = block(hash_in(s, rk), rk);
     return make_uint4(xor3(o.x, rk.w[40], s.z), xor3(o.y, rk.w[41], s.w), xor3(o.z, rk.w[42], s.z) ^ s.x,
                       xor3(o.w, rk.w[43], s.w) ^ s.y);
+  }
+  __device__ __forceinline__ uint4 prf(const AesRK &kd, uint32_t gate, uint32_t field, uint64_t idx) const {
+    return enc(make_uint4(uint32_t(idx), uint32_t(idx >> 32), field, gate), kd);
   }
 };
 
@@ -604,10 +613,18 @@ struct AesSel<2, 32> {
 template <int NT, int REP>
 using AesLds = typename AesSel<NT, REP>::type;
 
+// The table type of kernels that draw PRF blocks one by one.
+template <int NT, int REP>
+using AesPrf = std::conditional_t<std::is_same<AesLds<NT, REP>, AesPerm2>::value, AesPerm2Few, AesLds<NT, REP>>;
+
+// Table types whose enc2 and hash2 run two blocks side by side
+template <class A>
+constexpr bool kTwoChains = std::is_base_of<AesPerm2, A>::value || std::is_same<A, AesPerm>::value;
+
 // Two dealer PRF blocks of one key, side by side where the table type can.
 template <class A>
 __device__ __forceinline__ void enc_pair(const A &aes, const AesRK &k, uint4 u, uint4 v, uint4 *eu, uint4 *ev) {
-  if constexpr (std::is_same<A, AesPerm2>::value || std::is_same<A, AesPerm>::value) {
+  if constexpr (kTwoChains<A>) {
     aes.enc2(u, v, k, eu, ev);
   } else {
     *eu = aes.enc(u, k);

@@ -82,7 +82,7 @@ __device__ __forceinline__ uint32_t dcf_eval_walk(const A &aes, uint4 s, int m, 
 // the other on the other layouts.
 template <class A>
 __device__ __forceinline__ void hash_pair(const A &aes, uint4 s, uint4 u, const AesRK &rk, uint4 *hs, uint4 *hu) {
-  if constexpr (std::is_same<A, AesPerm2>::value || std::is_same<A, AesPerm>::value) {
+  if constexpr (kTwoChains<A>) {
     aes.hash2(s, u, rk, hs, hu);
   } else {
     *hs = aes.hash(s, rk);

@@ -1327,7 +1327,7 @@ template <typename T, int NT, int REP>
 __global__ void k_tr_expand(TrArgs<T> a, AesRK kp, int p) {
   __shared__ __align__(16) uint32_t lds[AesLds<NT, REP>::kWords];
   AesLds<NT, REP>::fill(lds);
-  AesLds<NT, REP> aes(lds);
+  AesPrf<NT, REP> aes(lds);
   uint8_t *w = a.w0;
   const size_t stride = size_t(gridDim.x) * blockDim.x;
   const int ncase = a.ncase;
