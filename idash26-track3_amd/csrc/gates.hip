@@ -331,8 +331,8 @@ __device__ __forceinline__ void tr_eval_both(const TrArgs<T> &a, const TrArgs<T>
 // lane's words of the roots, leaves and first correction words of its planes,
 // the mask bits, the lane's entry of the G table (lane j holds case j and, for
 // eight cases, 4 + j) and the kappa share.  A launch of few waves waits out every
-// load, so all go out at once, and those of a second gate (or a tree's next
-// level) while the first one runs.
+// load, so all go out at once, and those of a pair's second gate before the first
+// one runs.
 template <typename T>
 struct QuadKeys {
   uint32_t sa = 0, la = 0, ca = 0, za = 0, sb = 0, lb = 0, cb = 0, zb = 0;
@@ -573,8 +573,7 @@ __global__ void k_tr_eval_pool_tail_q(TrTail<T> t) {
 // The one-lane kernels' instances.  kFew: a CU has few waves (tr_few), whose walks
 // take the scheduler's order of reads (AesPerm2Few); kMid: the phases; kWide: 1024
 // threads in 64 registers, so that two such workgroups fit a CU (2 spilled, 8 in
-// Z_2^64: outside the level loops, but each a memory latency, 0.5 us, in a launch of
-// few waves).  All launches in the 64 registers and the phases, against now: RELUs
+// Z_2^64: some 0.5 us in a launch of few waves).  All launches in the 64 registers and the phases, against now: RELUs
 // of 79 elements per CU 57.1 -> 46.6 us (Z_2^64 107.6 -> 85.9), of 256 57.5 -> 55.6
 // (108.2 -> 105.2), 6-call TRMODs of 129 to 512 26.5-34.1 -> 25.9-33.3.
 enum { kFew, kMid, kWide };
@@ -782,8 +781,9 @@ __device__ __forceinline__ void tr_gen_tile(const Aes &aes, ConstWord *keys, con
 // 4160, the PRF blocks the rest) and, for few elements, by the chain of blocks a
 // thread runs one after another: each pair of PRF blocks of one key and the two
 // parties' hashes of a level run as two chains, which halves that chain and keeps
-// 32 reads in flight.  1.4 M EXTRELU elements 620 -> 535 us, 262144 132 -> 105,
-// 1024 74 -> 42 (one block at a time, and 112 registers spilled, before).
+// 32 reads in flight.  1.4 M EXTRELU elements 561 -> 526 us on changing inputs (619
+// -> 530 on the same ones again), 262144 132 -> 105, 1000 74 -> 41 (one block at a
+// time, and 110 registers spilled, before).
 template <typename T, int NT, int REP>
 __global__ void __launch_bounds__(1024, 4) k_tr_keygen(TrGenArgs<T> ka) {
   __shared__ __align__(16) uint32_t lds[AesLds<NT, REP>::kWords];
@@ -1034,9 +1034,9 @@ static int both_block(const Launch &L, const TrArgs<T> &a) {
   if (L.aes_block != 0 || aes > L.both_aes) return 0;
   return a.N >= size_t(L.num_cu) * size_t(L.both_min) ? 1024 : 0;
 }
-// Waves per SIMD of a both-party launch.  Eight (64 registers, a few spilled
-// outside the level loops; two workgroups per CU) keep the LDS reading at 98% of
-// its rate, but a round of the grid is then 2048 elements per CU: from 4096 on
+// Waves per SIMD of a both-party launch.  Eight (64 registers, 28 spilled, 35 in the
+// max-pool form, against 88 and 95 for four; two workgroups per CU) keep the LDS
+// reading at 97% of its rate, but a round of the grid is then 2048 elements per CU: from 4096 on
 // that is worth it (8192 per CU: 1037 against 1072 us for four waves; 1536: 261
 // against 204).  Beside other streams' launches four (one workgroup per CU) leave
 // those the other half of the CU: affinity B = 64 in 3 lanes 5.17 against 5.27 ms,

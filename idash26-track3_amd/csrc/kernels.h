@@ -35,7 +35,8 @@ struct Launch {
   int both_aes = kBothAesAlone;
   int both_min = kBothMinAlone;
   // Other streams' launches run beside this one's: a both-party launch then
-  // leaves half of a CU's wave slots and LDS to them (both_waves).
+  // leaves half of a CU's wave slots and LDS to them (both_waves), and a max-pool
+  // level stays in one-lane workgroups.
   bool shared = false;
   // Launches of a profiled forward use a separately named instantiation of the
   // DCF-evaluation kernel (same code), so kernel traces can tell them apart.
